@@ -3,8 +3,10 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload c3] [--channels N]
 
-One step = one loopback exchange of all cp logical ranks of the workload
-(payload read + FIFO write + FIFO read + output write), inputs resident in HBM.
+One step = one loopback exchange of all cp logical ranks of the workload through
+the LL128 FIFOs (payload read + FIFO write + FIFO read + output write), inputs
+resident in HBM; `direct` is the same call without a channel count, which copies
+between the ranks' tensors.
 Prints ONE JSON line: effective GB/s (algorithmic bytes / time per call) and
 microseconds per call; the roofline fraction of the kernel measured with HIP
 events on the launch stream, once with one set of tensors reused every step
@@ -333,9 +335,9 @@ def exchange_kernel_timing(w, steps: int = 200, warmup: int = 30):
     nbytes = w.exchange_bytes(channels)
     tensor_bytes = sum(t.numel() * t.element_size() for t in ins_o + ins_s) * 2
     n_sets = max(2, -(-(1 << 30) // tensor_bytes))
-    plans = [_ops.LoopbackPlan(ins_o, ins_s, ws)]
+    plans = [_ops.LoopbackPlan(ins_o, ins_s, ws, channels)]  # a channel count: the FIFO protocol
     hot = _event_us(plans[0].run, steps, warmup)
-    plans += [_ops.LoopbackPlan([t.clone() for t in ins_o], [t.clone() for t in ins_s], ws) for _ in range(n_sets - 1)]
+    plans += [_ops.LoopbackPlan([t.clone() for t in ins_o], [t.clone() for t in ins_s], ws, channels) for _ in range(n_sets - 1)]
     turn = [0]
 
     def next_set():
@@ -545,13 +547,16 @@ def main() -> int:
         pairs = [as_head_layout(w, o, s) for o, s in zip(ins_o, ins_s)]
         ins_o, ins_s = [p[0] for p in pairs], [p[1] for p in pairs]
         entries = w.tokens * w.heads_per_rank
-    def make_plan(o, s_):
+    channels = args.channels or _ops.auto_channel_count(w.cp, entries)
+
+    # The metric is the LL128 protocol's traffic, so the timed calls name the channel count; calls that leave it to the
+    # library copy between the ranks' tensors directly (`direct` below).
+    def make_plan(o, s_, n_channels=channels):
         if args.combine:
-            return _ops.CombinePlan(o, s_, ws, _ops.STATS_MAX_SUM, False, args.channels)
-        return _ops.LoopbackPlan(o, s_, ws, args.channels)
+            return _ops.CombinePlan(o, s_, ws, _ops.STATS_MAX_SUM, False, n_channels)
+        return _ops.LoopbackPlan(o, s_, ws, n_channels)
 
     plan = make_plan(ins_o, ins_s)
-    channels = args.channels or _ops.auto_channel_count(w.cp, entries)
     # algorithmic bytes: payload read + lines written + lines read + output written, with the lines this
     # channel count makes (the messages of a run are packed piece by piece, whole lines per run)
     per_head = args.layout == "head"
@@ -641,6 +646,24 @@ def main() -> int:
                 "us_per_call": cold_wall * 1e6 / roofline_steps}
         del plans
 
+    # The call as a program makes it, no channel count given: the same result without the FIFOs.
+    useful_bytes = (w.payload_bytes + w.cp * w.tokens * w.field0_bytes) if args.combine else 2 * w.payload_bytes
+    direct_us = _event_us(make_plan(ins_o, ins_s, 0).run, MIN_ROOFLINE_STEPS, 30)
+    direct = {"us_per_call": direct_us, "bytes_per_call": useful_bytes, "GBps": useful_bytes / direct_us / 1e3,
+              "note": "channel_count 0: payload read + result written, nothing through the FIFOs; HIP events, one set of tensors"}
+    if n_sets >= 2 and graph is None:
+        plans = [make_plan([t.clone() for t in ins_o], [t.clone() for t in ins_s], 0) for _ in range(n_sets)]
+        turn = [0]
+
+        def next_set():
+            plans[turn[0] % n_sets].run()
+            turn[0] += 1
+
+        direct["us_per_call_cold"] = _event_us(next_set, MIN_ROOFLINE_STEPS, n_sets)
+        direct["GBps_cold"] = useful_bytes / direct["us_per_call_cold"] / 1e3
+        del plans
+    status |= _ops.device_status()
+
     ok = status == 0
     if not args.no_check and args.combine:
         import numpy as np
@@ -669,8 +692,6 @@ def main() -> int:
     achieved = bytes_per_call / (avg_kernel_ms * 1e-3) / 1e9
     kernel_name = "helix_combine_kernel" if args.combine else "helix_exchange_kernel"
     traffic = None if args.layout == "head" else MEASURED_TRAFFIC_BYTES.get((kernel_name, w.name, channels))
-    # the exchange as a user sees it: payload in, payload out (a direct permuted copy would move just that)
-    useful_bytes = (w.payload_bytes + w.cp * w.tokens * w.field0_bytes) if args.combine else 2 * w.payload_bytes
     result = {
         "metric": METRIC,
         "value": bytes_per_call / (ms_per_step * 1e-3) / 1e9,
@@ -727,6 +748,7 @@ def main() -> int:
             "achieved_cold": None if cold is None else bytes_per_call / (cold["kernel_us"] * 1e-6) / 1e9,
         },
         "cold": cold,
+        "direct": direct,
     }
     if not args.no_host_timing and not args.combine and args.layout == "token" and graph is None:
         result["host_us_per_call"] = host_timing(w, ws, ins_o, ins_s)

@@ -63,11 +63,11 @@ def main() -> int:
     for r in range(w.cp):
         helix_a2a.init_workspace(ws, r, w.cp)
     ins_o, ins_s = make_inputs(w, "cuda")
-    if args.combine:
-        plan = _ops.CombinePlan(ins_o, ins_s, ws, _ops.STATS_MAX_SUM, False, args.channels)
-    else:
-        plan = _ops.LoopbackPlan(ins_o, ins_s, ws, args.channels)
     channels = args.channels or _ops.auto_channel_count(w.cp, w.tokens)
+    if args.combine:
+        plan = _ops.CombinePlan(ins_o, ins_s, ws, _ops.STATS_MAX_SUM, False, channels)
+    else:
+        plan = _ops.LoopbackPlan(ins_o, ins_s, ws, channels)
     streams = w.cp * w.cp * channels
     max_waves = 1 << 16
     buf = np.zeros((max_waves, 4), dtype=np.uint64)

@@ -15,7 +15,7 @@ import sys
 from pathlib import Path
 
 HERE = Path(__file__).resolve().parent
-SOURCES = [HERE / "csrc" / "helix_kernels.hip", HERE / "csrc" / "helix_c_api.hip"]
+SOURCES = [HERE / "csrc" / "helix_kernels.hip", HERE / "csrc" / "helix_direct.hip", HERE / "csrc" / "helix_c_api.hip"]
 OUTPUT = HERE / "helix_a2a" / "libhelix_a2a.so"
 
 HIPCC_FLAGS = [

@@ -15,7 +15,7 @@
 #include <mutex>
 
 #include "../../include/helix_a2a.h"
-#include "helix_kernels.hpp"
+#include "helix_direct.hpp"
 
 namespace {
 
@@ -79,6 +79,7 @@ struct DeviceState {
   hipError_t initError = hipSuccess;
   int cuCount = 0;
   uint32_t* status = nullptr;  // device status word
+  const uint64_t* never = nullptr;  // a device word that stays zero
   uint8_t* scratch = nullptr;  // this device's copy of the built-in workspace (helix_a2a_alltoall_loopback_static)
   std::mutex scratchMutex;
   int scratchCp = 0;           // cp_size the built-in workspace is laid out and initialised for (0 = not yet)
@@ -86,8 +87,8 @@ struct DeviceState {
 };
 DeviceState g_devices[kMaxDevices];
 
-// status word: one per device, lives until the process ends
-__device__ uint32_t g_statusWord[4];
+// word 0: status, one per device, lives until the process ends; words 2 and 3 stay zero
+__device__ __align__(16) uint32_t g_statusWord[4];
 
 // Built-in workspace of helix_a2a_alltoall_loopback_static: room for kStaticStreams FIFOs
 // (sender, receiver, channel) with their two counter blocks, 64.06 MiB, held by every device the
@@ -111,6 +112,7 @@ int device_state(DeviceState** out) {
     st.initError = hipGetSymbolAddress(&p, HIP_SYMBOL(g_statusWord));
     if (st.initError != hipSuccess) return;
     st.status = static_cast<uint32_t*>(p);
+    st.never = reinterpret_cast<const uint64_t*>(st.status + 2);
     st.initError = hipMemset(st.status, 0, sizeof(uint32_t) * 4);
     if (st.initError != hipSuccess) return;
     void* sp = nullptr;
@@ -178,6 +180,7 @@ struct Plan {
   int roundEntries;  // entries per stream-ordered round (multiple of runChannels)
   MsgShape shape;
   int cuCount;
+  bool wire;  // the caller names a channel count or a setting of the FIFO protocol: the exchange goes through the FIFOs
 };
 
 int check_field(const helix_a2a_field_t& f, const char* name, int eltSize, int entryCount, int cpSize,
@@ -294,6 +297,7 @@ int build_plan(const helix_a2a_params_t* ranks, int count, bool exchangeOutputs,
     return fail(HELIX_A2A_ERR_INVALID_ARGUMENT, "a FIFO region of %d x %d streams is beyond what the kernels address", cp, maxCh);
 
   int channels = p0.channel_count > 0 ? p0.channel_count : env_channel_count();
+  plan->wire = channels > 0 || g_singleRound.load() != 0 || g_unitsPerWavefront.load() != -1 || g_teamUnits.load() != -1;
   if (channels > maxCh) {
     if (p0.channel_count > 0 || builtin == nullptr)
       return fail(HELIX_A2A_ERR_INVALID_ARGUMENT, "channel_count %d exceeds max_channel_count %d", channels, maxCh);
@@ -369,6 +373,18 @@ int launch_rounds(Plan& plan, bool send, bool recv, bool allowRounds, hipStream_
     HELIX_HIP_TRY(launch_exchange(a, units_per_part(), max_parts_for(a, plan.cuCount), team_units(), stream));
   }
   return HELIX_A2A_OK;
+}
+
+// All ranks of one device in one call. Every tensor is in reach of one launch, so nothing has to travel through the
+// FIFOs; they are used where the caller pins how (a channel count, in the descriptor or the environment, or a setting
+// of the protocol), which is a request for that traffic. `broken`: the word that stops exchanges on a broken workspace.
+int launch_all_ranks(Plan& plan, const uint64_t* broken, hipStream_t stream) {
+  if (plan.wire) return launch_rounds(plan, true, true, true, stream);
+  HELIX_HIP_TRY(launch_direct_exchange(plan.args, broken, stream));
+  return HELIX_A2A_OK;
+}
+const uint64_t* broken_word(const KernelArgs& a) {
+  return reinterpret_cast<const uint64_t*>(a.workspace + broken_word_offset(a.cpSize, a.maxChannels));
 }
 
 // Wait for `stream`, read the device status word and clear it. Everything is ordered on `stream` itself (nothing
@@ -477,7 +493,7 @@ int helix_a2a_alltoall_loopback(const helix_a2a_params_t* per_rank, int cp_size,
   Plan plan;
   int rc = build_plan(per_rank, cp_size, true, &plan);
   if (rc) return rc;
-  return finish_call(launch_rounds(plan, true, true, true, static_cast<hipStream_t>(stream)), static_cast<hipStream_t>(stream));
+  return finish_call(launch_all_ranks(plan, broken_word(plan.args), static_cast<hipStream_t>(stream)), static_cast<hipStream_t>(stream));
 }
 
 int helix_a2a_alltoall_loopback_static(const helix_a2a_params_t* per_rank, int cp_size, int reset, void* stream) {
@@ -500,7 +516,7 @@ int helix_a2a_alltoall_loopback_static(const helix_a2a_params_t* per_rank, int c
   Plan plan;
   if ((rc = build_plan(per_rank, cp_size, true, &plan, &ws))) return rc;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  {
+  if (plan.wire || reset) {
     // The array keeps the last call's contents. Its layout depends on cp_size, so a change of cp_size
     // (or the first call, or a caller's request) lays it out again: FIFO bytes 0xFF, counters 0, by a
     // fill kernel in stream order ahead of the exchange.
@@ -519,7 +535,8 @@ int helix_a2a_alltoall_loopback_static(const helix_a2a_params_t* per_rank, int c
       st->scratchCp = cp_size;
     }
   }
-  return finish_call(launch_rounds(plan, true, true, true, s), s);
+  // An exchange that does not touch the array cannot break it and runs whatever state it is in.
+  return finish_call(launch_all_ranks(plan, st->never, s), s);
 }
 
 int helix_a2a_alltoall_combine_loopback(const helix_a2a_params_t* per_rank, const helix_a2a_combine_out_t* out,

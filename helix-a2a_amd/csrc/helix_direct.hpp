@@ -1,0 +1,43 @@
+// helix_direct.hpp -- launch descriptors of the direct kernels (internal; the
+// public boundary is include/helix_a2a.h).
+//
+// When all cp ranks of an exchange are logical ranks of one device and their
+// calls are issued as one launch, every send tensor is complete before the
+// launch starts and every receive tensor is addressable from it. Nothing then
+// has to travel through a FIFO: a launch reads each send row once and writes it
+// where it belongs, half the bytes of the same exchange through LL128 lines.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "helix_kernels.hpp"
+
+namespace helix {
+
+struct DirectArgs {
+  RankPtrs rank[kMaxCpSize];
+  const uint64_t* broken;  // a launch that finds this word non-zero (the workspace's broken word) writes nothing
+  uint32_t* status;        // device status word (HELIX_A2A_STATUS_* bits)
+  int cpSize;
+  uint32_t sendStride0, sendStride1;  // bytes between consecutive (entry, peer) rows
+  uint32_t recvStride0, recvStride1;
+  uint32_t sendBytes0, recvBytes0;    // extent of each partial_o tensor (< 2 GiB), the range of its buffer descriptor
+  FastDiv byCp;
+  // partial_o: 16-byte units, a wavefront moves 64 consecutive ones ("chunk") of one (sender, receiver) pair
+  uint32_t units;       // of one pair: entries * rowUnits
+  uint32_t rowUnits;    // of one row
+  FastDiv byRowUnits;
+  uint32_t waves;
+  uint32_t groupShift;  // 2^groupShift consecutive wavefronts take consecutive chunks of one pair
+  // softmax_stats: 8-byte pieces, all pairs together in the order (entry, receiver, sender, piece)
+  uint32_t pieces;
+  uint32_t rowPieces;
+  FastDiv byRowPieces;
+  uint32_t statsBlocks;  // workgroups that move statistics; they come first in the launch
+};
+
+// out[r][e, s, :] = in[s][e, r, :] for both fields and all ranks of `a`.
+hipError_t launch_direct_exchange(const KernelArgs& a, const uint64_t* broken, hipStream_t stream);
+
+}  // namespace helix

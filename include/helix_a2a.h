@@ -184,10 +184,16 @@ int helix_a2a_alltoall_recv(const helix_a2a_params_t* per_rank, int rank_count, 
 /*
  * Loopback exchange: all cp_size logical ranks of one device in a single
  * fused launch. per_rank[r] must have cp_rank == r; all descriptors share
- * workspace, shapes and strides. Sender wavefronts are placed before receiver
- * wavefronts in dispatch order. channel_count is taken from per_rank[0].
+ * workspace, shapes and strides. channel_count is taken from per_rank[0].
  * After the stream drains, recv of rank r holds
  *   recv_r[e, s, :] = send_s[e, r, :]     for both fields.
+ * With channel_count 0 (and no HELIX_A2A_CHANNEL_COUNT, and the settings of the
+ * protocol below at their defaults) nothing goes through the FIFOs: every
+ * rank's memory is in reach of the one launch, which copies each row to its
+ * place. A caller that names a channel count gets the FIFO protocol over that
+ * many channels, sender wavefronts ahead of receiver wavefronts in dispatch
+ * order, at twice the memory traffic. Both may alternate on one workspace, and
+ * both do nothing on a broken one.
  */
 int helix_a2a_alltoall_loopback(const helix_a2a_params_t* per_rank, int cp_size, void* stream);
 
@@ -200,7 +206,9 @@ int helix_a2a_alltoall_loopback(const helix_a2a_params_t* per_rank, int cp_size,
  * HELIX_A2A_STATIC_MAX_STREAMS x (512 KiB + 512 B) = 67 174 400 bytes that
  * every GPU the library runs on holds until the process ends. The workspace
  * members of the descriptors must be NULL / 0 (max_channel_count is ignored);
- * everything else is as for helix_a2a_alltoall_loopback, same results.
+ * everything else is as for helix_a2a_alltoall_loopback, same results. With
+ * channel_count 0 the call does not touch the array at all (unless `reset` asks
+ * for it to be laid out again), and of the following only the limit on cp_size applies.
  *   limit   cp_size * cp_size <= HELIX_A2A_STATIC_MAX_STREAMS, i.e. cp_size <= 11
  *           (HELIX_A2A_ERR_CAPACITY beyond); the channel count is at most
  *           128 / cp_size^2, so large exchanges run slower than with a full workspace.
