@@ -589,6 +589,10 @@ int helix_a2a_alltoall_combine_loopback(const helix_a2a_params_t* per_rank, cons
     a.rank[r].recv1 = reinterpret_cast<uint8_t*>(out[r].lse_out);
   }
   if (plan.entryCount == 0) return HELIX_A2A_OK;
+  if (!plan.wire) {  // see launch_all_ranks
+    HELIX_HIP_TRY(launch_direct_combine(a, broken_word(a), static_cast<hipStream_t>(stream)));
+    return finish_call(HELIX_A2A_OK, static_cast<hipStream_t>(stream));
+  }
   for (int begin = 0; begin < plan.entryCount; begin += plan.roundEntries) {
     a.entryBegin = begin;
     long end = static_cast<long>(begin) + plan.roundEntries;

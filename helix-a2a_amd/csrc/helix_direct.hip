@@ -8,12 +8,10 @@
 // 83 -> 46 us (5.9 TB/s, a plain copy of 1 GiB reaches 6.2), cp = 16, T = 1024,
 // rows of 512 bytes 93 -> 43 us.
 #include "helix_direct.hpp"
+#include "helix_element.hpp"
 
 namespace helix {
 namespace {
-
-using u32x2 = uint32_t __attribute__((ext_vector_type(2)));
-using u32x4 = uint32_t __attribute__((ext_vector_type(4)));
 
 // buffer cache-policy immediates: bit 0 sc0, bit 1 nt, bit 4 sc1
 constexpr int kAuxNone = 0;
@@ -30,11 +28,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, ui
 }
 
 // Whether the workspace was broken before this launch, read through the scalar cache (empty at every launch).
-__device__ __forceinline__ bool broken_at_launch(const DirectArgs& a) {
+__device__ __forceinline__ bool broken_at_launch(const DirectRanks& a) {
   using ConstWord = const __attribute__((address_space(4))) uint64_t;
   return *reinterpret_cast<ConstWord*>(reinterpret_cast<uintptr_t>(a.broken)) != 0;
 }
-__device__ __forceinline__ void report_broken(const DirectArgs& a) {
+__device__ __forceinline__ void report_broken(const DirectRanks& a) {
   if (threadIdx.x % kWaveLanes == 0) atomicOr(a.status, kStatusBrokenWorkspace);
 }
 
@@ -46,12 +44,12 @@ using GlobalPiece = __attribute__((address_space(1))) u32x2;
 // pairs share are fetched by one L2 and written from one L2, and every store covers cp consecutive rows of the
 // receiver. The rank is a lane's own then; the 2 * cp pointers go through LDS.
 template <int kPerThread>
-__device__ __forceinline__ void move_statistics(const DirectArgs& a, uint64_t (&from)[kMaxCpSize], uint64_t (&to)[kMaxCpSize]) {
-  const int tid = static_cast<int>(threadIdx.x);
+__device__ __forceinline__ void move_statistics(const DirectExchangeArgs& a, uint64_t (&from)[kMaxCpSize], uint64_t (&to)[kMaxCpSize]) {
+  const uint32_t tid = threadIdx.x;
   uint64_t mineFrom = 0, mineTo = 0;
-  for (int base = 0; base < a.cpSize; base += 8) {
+  for (uint32_t base = 0; base < a.cpSize; base += 8) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {  // eight ranks' pointers in one trip to the scalar cache
+    for (uint32_t i = 0; i < 8; ++i) {  // eight ranks' pointers in one trip to the scalar cache
       const uint64_t f = reinterpret_cast<uint64_t>(a.rank[base + i].send1), t = reinterpret_cast<uint64_t>(a.rank[base + i].recv1);
       if (tid == base + i) {
         mineFrom = f;
@@ -95,7 +93,7 @@ __device__ __forceinline__ void move_statistics(const DirectArgs& a, uint64_t (&
 // shorter than an access, a workgroup takes four consecutive accesses of one pair instead (cp = 16 rows of 512 bytes
 // 46.3 -> 43.7 us; rows of 2 KiB stay with the receivers side by side: 512 tokens per rank more 44.9 -> 48.0 us).
 template <int kStatsPerThread, int kAuxLoad, int kAuxStore>
-__global__ __launch_bounds__(kBlockThreads) void helix_direct_exchange_kernel(DirectArgs a) {
+__global__ __launch_bounds__(kBlockThreads) void helix_direct_exchange_kernel(DirectExchangeArgs a) {
   __shared__ uint64_t from[kMaxCpSize], to[kMaxCpSize];
   if (blockIdx.x < a.statsBlocks) return move_statistics<kStatsPerThread>(a, from, to);
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWaveLanes);
@@ -118,15 +116,188 @@ __global__ __launch_bounds__(kBlockThreads) void helix_direct_exchange_kernel(Di
   __builtin_amdgcn_raw_buffer_store_b128(v, out, live ? (e * a.cpSize + s) * a.recvStride0 + off : kOutOfRange, 0, kAuxStore);
 }
 
+// ---------------------------------------------------------------------------
+// combine
+// ---------------------------------------------------------------------------
+// The exchange and the combine after it in one pass: a lane makes one piece of one rank's output from the cp pieces
+// of the senders' tensors that belong to it, so an input row is read once and only the weighted sum is written.
+// Bound by the reads (cp input bytes for one written); no FIFO lines: cp = 8, T = 256, 8 heads of 128 per rank
+// 20.9 -> 6.6 us, T = 128, 16 heads of 512 71 -> 27 us (5.6 TB/s), cp = 16, T = 1024, 2 heads of 128 73 -> 27.6 us.
+
+// Pieces of kWords * 2 elements.
+template <int kDtype, int kWords>
+struct Piece;
+template <int kDtype>
+struct Piece<kDtype, 4> {
+  using Raw = u32x4;
+  template <int kAux>
+  static __device__ __forceinline__ Raw load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kAux);
+  }
+  template <int kAux>
+  static __device__ __forceinline__ void store(const float (&f)[8], __amdgpu_buffer_rsrc_t r, uint32_t off) {
+    const float lo[4] = {f[0], f[1], f[2], f[3]}, hi[4] = {f[4], f[5], f[6], f[7]};
+    const u32x2 x = narrow_piece<kDtype>(lo), y = narrow_piece<kDtype>(hi);
+    __builtin_amdgcn_raw_buffer_store_b128(u32x4{x.x, x.y, y.x, y.y}, r, off, 0, kAux);
+  }
+  static __device__ __forceinline__ void accumulate(float (&acc)[8], float w, Raw v) {
+    float lo[4], hi[4];
+    widen4<kDtype>(u32x2{v.x, v.y}, lo);
+    widen4<kDtype>(u32x2{v.z, v.w}, hi);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      acc[c] += w * lo[c];
+      acc[4 + c] += w * hi[c];
+    }
+  }
+};
+template <int kDtype>
+struct Piece<kDtype, 2> {
+  using Raw = u32x2;
+  template <int kAux>
+  static __device__ __forceinline__ Raw load(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, kAux);
+  }
+  template <int kAux>
+  static __device__ __forceinline__ void store(const float (&f)[4], __amdgpu_buffer_rsrc_t r, uint32_t off) {
+    __builtin_amdgcn_raw_buffer_store_b64(narrow_piece<kDtype>(f), r, off, 0, kAux);
+  }
+  static __device__ __forceinline__ void accumulate(float (&acc)[4], float w, Raw v) {
+    float f[4];
+    widen4<kDtype>(v, f);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) acc[c] += w * f[c];
+  }
+};
+
+// A wavefront makes 64 consecutive pieces of one rank's output (one per lane: two per lane measured the same at
+// large sizes and up to 25 % slower below, where wavefronts are few); consecutive wavefronts take consecutive ranks,
+// whose rows are neighbours in every input tensor.
+//
+// Weights are worked out once per wavefront and head, not per lane: the wavefront turns sideways, lane i serves the
+// (i / G)-th head the pieces touch ("slot") and sender i % G, loads that sender's log-sum-exp of that head, and a
+// softmax over the G lanes of the slot gives the weights, which go through LDS to the lanes that own pieces of the
+// head. G = 4, 8, 16 or 32 lanes serve a slot for up to as many ranks. The payload loads are behind the statistics
+// loads and in front of the softmax, up to eight ranks' pieces in flight (sixteen at a time for sixteen ranks: the same).
+template <int kDtype, int kLanesPerSlot, int kWords, int kAuxLoad, int kAuxStore>
+__global__ __launch_bounds__(kBlockThreads) void helix_direct_combine_kernel(DirectCombineArgs a) {
+  using P = Piece<kDtype, kWords>;
+  constexpr uint32_t kPieceSize = kWords * 4;
+  constexpr uint32_t kElements = kWords * 2;
+  constexpr int kMaxSlots = kWords == 4 ? 17 : 9;  // heads that 64 pieces touch: a head is 32 elements or more
+  constexpr uint32_t kSlotsPerPass = kWaveLanes / kLanesPerSlot;
+  constexpr int kGroup = kLanesPerSlot < 8 ? kLanesPerSlot : 8;
+  __shared__ float __attribute__((aligned(16))) weights[kBlockWaves][kMaxSlots][kLanesPerSlot];
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWaveLanes);
+  const uint32_t lane = threadIdx.x % kWaveLanes;
+  const uint32_t w = blockIdx.x * kBlockWaves + wave;
+  if (w >= a.waves) return;
+  const uint32_t chunk = fast_div_by(w, a.byCp);
+  const uint32_t r = w - chunk * a.cpSize;
+  const bool broken = broken_at_launch(a);
+  const uint32_t first = chunk * kWaveLanes;
+  const uint32_t last = min(first + kWaveLanes, a.outPieces) - 1u;
+  const uint32_t firstHead = fast_div_by(first, a.byHeadPieces);  // heads are counted through the rows: entry * heads + head
+  const uint32_t slots = fast_div_by(last, a.byHeadPieces) - firstHead + 1u;
+
+  // ---- statistics of the first slots
+  const uint32_t q = lane % kLanesPerSlot;  // the sender this lane serves
+  const bool realSender = q < a.cpSize;
+  uint64_t stats = 0;
+#pragma unroll
+  for (int i = 0; i < kLanesPerSlot; ++i) {
+    const uint64_t p = reinterpret_cast<uint64_t>(a.rank[i].send1);
+    if (q == static_cast<uint32_t>(i)) stats = p;
+  }
+  auto load_statistics = [&](uint32_t slot, uint32_t& e, uint32_t& h) -> u32x2 {
+    const uint32_t head = firstHead + slot;
+    e = fast_div_by(head, a.byHeads);
+    h = head - e * a.heads;
+    u32x2 v = {0u, 0u};
+    if (slot < slots && realSender) {
+      const uint64_t row = stats + (e * a.cpSize + r) * a.sendStride1;
+      if (a.statsMode == 2)  // one log-sum-exp per head
+        v.x = *reinterpret_cast<const __attribute__((address_space(1))) uint32_t*>(row + h * 4u);
+      else
+        v = *reinterpret_cast<const GlobalPiece*>(row + h * 8u);
+    }
+    return v;
+  };
+  uint32_t slot = lane / kLanesPerSlot, e, h;
+  u32x2 sv = load_statistics(slot, e, h);
+
+  // ---- the pieces of the first ranks
+  const uint32_t p = first + lane;
+  const bool live = p < a.outPieces;
+  const uint32_t myHead = fast_div_by(p, a.byHeadPieces);
+  const uint32_t myEntry = fast_div_by(myHead, a.byHeads);
+  const uint32_t mySlot = live ? myHead - firstHead : 0u;
+  const uint32_t from = live ? (myEntry * a.cpSize + r) * a.sendStride0 + (p - myEntry * a.rowPieces) * kPieceSize : kOutOfRange;
+  typename P::Raw v[kGroup];
+  auto load_group = [&](int g) {
+#pragma unroll
+    for (int i = 0; i < kGroup; ++i) {
+      // beyond cp: a descriptor of no bytes, zeros without memory traffic
+      const __amdgpu_buffer_rsrc_t in = make_rsrc(a.rank[g + i].send0, static_cast<uint32_t>(g + i) < a.cpSize ? a.sendBytes0 : 0u);
+      v[i] = P::template load<kAuxLoad>(in, from);
+    }
+  };
+  load_group(0);
+
+  // ---- weights
+  for (uint32_t base = 0; base < slots; base += kSlotsPerPass) {
+    if (base > 0) {
+      slot = base + lane / kLanesPerSlot;
+      sv = load_statistics(slot, e, h);
+    }
+    const bool serving = slot < slots && realSender;
+    const float lse = serving ? lse_of_stats(sv.x, sv.y, a.statsMode == 2 ? 0 : a.statsMode, 0, a.lseBase2 != 0) : -INFINITY;
+    float m = lse;
+#pragma unroll
+    for (int x = 1; x < kLanesPerSlot; x <<= 1) m = fmaxf(m, shuffle_xor(m, x));
+    if (m == -INFINITY) m = 0.0f;  // every rank masked: weights 0, log-sum-exp -inf
+    float ex = fast_exp(lse - m);
+    if (isnan(ex)) ex = 0.0f;
+    float total = ex;
+#pragma unroll
+    for (int x = 1; x < kLanesPerSlot; x <<= 1) total += shuffle_xor(total, x);
+    // (ranks beyond cp get weight 0: their pieces are zeros, and 0 * 0 stays 0)
+    if (slot < slots) weights[wave][slot][q] = ex * __builtin_amdgcn_rcpf(fmaxf(total, 1e-10f));
+    float* lseOut = reinterpret_cast<float*>(a.rank[r].recv1);
+    if (lseOut != nullptr && serving && q == 0 && !broken) {  // (a head that two wavefronts share gets the same value twice)
+      const float combinedLse = fast_log(total) + m;
+      lseOut[static_cast<uint64_t>(e) * a.heads + h] = a.lseBase2 ? combinedLse * 1.4426950408889634f : combinedLse;
+    }
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+  // ---- the weighted sum
+  float acc[kElements];
+#pragma unroll
+  for (uint32_t c = 0; c < kElements; ++c) acc[c] = 0.0f;
+#pragma unroll
+  for (int g = 0; g < kLanesPerSlot; g += kGroup) {
+    if (g > 0) load_group(g);
+    const float* wq = &weights[wave][mySlot][g];
+#pragma unroll
+    for (int i = 0; i < kGroup; ++i) P::accumulate(acc, wq[i], v[i]);
+  }
+  if (broken) return report_broken(a);
+  P::template store<kAuxStore>(acc, make_rsrc(a.rank[r].recv0, a.recvBytes0), live ? p * kPieceSize : kOutOfRange);
+}
+
 }  // namespace
 
-// A launch that reads and writes more than this takes its payload past the memory-side cache (256 MB) on the way
-// in: what the previous kernels left there is mostly older than the inputs, or is not all of them, and a read that
-// does not allocate leaves room for the writes. Measured over inputs that were just written, over rotating sets,
-// and over three sets in rotation: 134 MB 20.2 -> 19.4, 25.2 -> 23.6, 19.8 -> 23.6 us; 168 MB 31.2 -> 23.8,
-// 29.8 -> 28.5, 27.6 -> 28.4; 201 MB 53.2 -> 28.9, 35.2 -> 33.3, 32.0 -> 33.4; 268 MB 55.4 -> 32.8, 47.0 -> 45.0,
-// 46.3 -> 44.9.
-constexpr uint64_t kStreamingBytes = 150ull << 20;
+// A launch that reads more payload than this takes it past the memory-side cache (256 MB) on the way in: what that
+// cache holds is older than the inputs, or not all of them, and a read that does not allocate leaves room for the
+// writes. Measured over inputs that were just written, over rotating sets, and over three sets in rotation:
+//   exchange  67 MB 20.2 -> 19.4, 25.2 -> 23.6, 19.8 -> 23.6 us; 84 MB 31.2 -> 23.8, 29.8 -> 28.5, 27.6 -> 28.4;
+//            101 MB 53.2 -> 28.9, 35.2 -> 33.3, 32.0 -> 33.4; 134 MB 55.4 -> 32.8, 47.0 -> 45.0, 46.3 -> 44.9
+//   combine   67 MB equal, 16.7 -> 15.5, 14.2 -> 15.3; 84 MB 20.5 -> 15.7, 19.7 -> 18.5, 17.4 -> 17.8;
+//            101 MB 29.1 -> 18.0, 23.9 -> 22.3, 22.3 -> 22.2; 134 MB 35.7 -> 19.4, 29.1 -> 27.4, 29.2 -> 26.8
+constexpr uint64_t kStreamingBytes = 75ull << 20;
 
 // Statistics pieces up to which a thread takes one piece instead of four: below, the launch waits for the chain of
 // one thread (pointers, load, store), not for memory (cp = 4, T = 64: 3.4 -> 2.7 us; an empty kernel takes 2.1).
@@ -135,23 +306,31 @@ constexpr uint32_t kShortStatsPieces = 65536;
 // Wavefronts of a launch, at most: larger exchanges go out as several launches of consecutive entries.
 constexpr uint64_t kMaxLaunchWaves = 1ull << 25;
 
-hipError_t launch_direct_exchange(const KernelArgs& a, const uint64_t* broken, hipStream_t stream) {
-  DirectArgs d{};
-  const uint32_t cp = static_cast<uint32_t>(a.cpSize);
+static void set_ranks(DirectRanks& d, const KernelArgs& a, const uint64_t* broken) {
+  for (int r = 0; r < a.cpSize; ++r) d.rank[r] = a.rank[r];
   d.broken = broken;
   d.status = a.status;
-  d.cpSize = a.cpSize;
+  d.cpSize = static_cast<uint32_t>(a.cpSize);
   d.sendStride0 = static_cast<uint32_t>(a.sendStride0);
   d.sendStride1 = static_cast<uint32_t>(a.sendStride1);
   d.recvStride0 = static_cast<uint32_t>(a.recvStride0);
   d.recvStride1 = static_cast<uint32_t>(a.recvStride1);
-  d.byCp = fast_div(cp);
+  d.sendBytes0 = a.sendBytes0;
+  d.recvBytes0 = a.recvBytes0;
+  d.byCp = fast_div(d.cpSize);
+}
+static bool streams_payload(const KernelArgs& a) { return static_cast<uint64_t>(a.cpSize) * a.sendBytes0 > kStreamingBytes; }
+
+hipError_t launch_direct_exchange(const KernelArgs& a, const uint64_t* broken, hipStream_t stream) {
+  DirectExchangeArgs d{};
+  set_ranks(d, a, broken);
+  const uint32_t cp = d.cpSize;
   d.rowUnits = static_cast<uint32_t>(a.field0Bytes) / kUnitBytes;
   d.byRowUnits = fast_div(d.rowUnits);
   d.rowPieces = static_cast<uint32_t>(a.field1Bytes) / kPieceBytes;
   d.byRowPieces = fast_div(d.rowPieces);
   d.groupShift = a.field0Bytes < kWaveLanes * kUnitBytes ? 2 : 0;
-  const bool streaming = cp * (static_cast<uint64_t>(a.sendBytes0) + a.recvBytes0) > kStreamingBytes;
+  const bool streaming = streams_payload(a);
   // Rows of whole 128-byte lines are written through (their lines are complete with one store: rows of 2 KiB 11.0 ->
   // 10.1 us, of 512 bytes 46.0 -> 43.5); others leave it to the L2 to put the halves of a line together (rows of 480
   // bytes 9.8 us written through, 9.2 left there).
@@ -193,6 +372,47 @@ hipError_t launch_direct_exchange(const KernelArgs& a, const uint64_t* broken, h
     if (err != hipSuccess) return err;
   }
   return hipSuccess;
+}
+
+template <int kDtype, int kWords, int kAuxLoad, int kAuxStore>
+static void launch_combine_kernel(const DirectCombineArgs& d, hipStream_t stream) {
+  const dim3 blocks((d.waves + kBlockWaves - 1) / kBlockWaves), threads(kBlockThreads);
+#define HELIX_LAUNCH_COMBINE(G) hipLaunchKernelGGL((helix_direct_combine_kernel<kDtype, G, kWords, kAuxLoad, kAuxStore>), blocks, threads, 0, stream, d)
+  if (d.cpSize <= 4) HELIX_LAUNCH_COMBINE(4);
+  else if (d.cpSize <= 8) HELIX_LAUNCH_COMBINE(8);
+  else if (d.cpSize <= 16) HELIX_LAUNCH_COMBINE(16);
+  else HELIX_LAUNCH_COMBINE(32);
+#undef HELIX_LAUNCH_COMBINE
+}
+
+template <int kDtype, int kWords>
+static void launch_combine_kernel(const DirectCombineArgs& d, bool streaming, hipStream_t stream) {
+  // a result that fits beside its inputs is written through (T = 256: 6.8 -> 6.5 us); one behind a stream of inputs is not
+  // (T = 128, 16 heads of 512: 27.1, written through 27.6)
+  if (streaming) launch_combine_kernel<kDtype, kWords, kAuxNt, kAuxNt>(d, stream);
+  else launch_combine_kernel<kDtype, kWords, kAuxNone, kAuxNtSc1>(d, stream);
+}
+
+hipError_t launch_direct_combine(const KernelArgs& a, const uint64_t* broken, hipStream_t stream) {
+  DirectCombineArgs d{};
+  set_ranks(d, a, broken);
+  const bool wide = a.headDim % 8 == 0;
+  const uint32_t pieceSize = wide ? 16 : 8;
+  d.rowPieces = static_cast<uint32_t>(a.field0Bytes) / pieceSize;
+  d.headPieces = static_cast<uint32_t>(a.headDim) * 2u / pieceSize;
+  d.heads = static_cast<uint32_t>(a.heads);
+  d.byHeadPieces = fast_div(d.headPieces);
+  d.byHeads = fast_div(d.heads);
+  d.outPieces = static_cast<uint32_t>(a.entryEnd) * d.rowPieces;
+  d.statsMode = a.statsMode;
+  d.lseBase2 = a.lseBase2;
+  d.waves = (d.outPieces + kWaveLanes - 1) / kWaveLanes * d.cpSize;  // at most 2^22: a rank's output is < 2 GiB / cp
+  const bool streaming = streams_payload(a);
+  if (a.dtype == 0)
+    wide ? launch_combine_kernel<0, 4>(d, streaming, stream) : launch_combine_kernel<0, 2>(d, streaming, stream);
+  else
+    wide ? launch_combine_kernel<1, 4>(d, streaming, stream) : launch_combine_kernel<1, 2>(d, streaming, stream);
+  return hipGetLastError();
 }
 
 }  // namespace helix

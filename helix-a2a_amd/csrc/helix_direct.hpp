@@ -15,20 +15,24 @@
 
 namespace helix {
 
-struct DirectArgs {
+// What both kernels know of the ranks' tensors.
+struct DirectRanks {
   RankPtrs rank[kMaxCpSize];
   const uint64_t* broken;  // a launch that finds this word non-zero (the workspace's broken word) writes nothing
   uint32_t* status;        // device status word (HELIX_A2A_STATUS_* bits)
-  int cpSize;
+  uint32_t cpSize;
   uint32_t sendStride0, sendStride1;  // bytes between consecutive (entry, peer) rows
   uint32_t recvStride0, recvStride1;
-  uint32_t sendBytes0, recvBytes0;    // extent of each partial_o tensor (< 2 GiB), the range of its buffer descriptor
+  uint32_t sendBytes0, recvBytes0;    // extent of each partial_o and result tensor (< 2 GiB), the range of its buffer descriptor
+  uint32_t waves;                     // wavefronts of the launch that move partial_o
   FastDiv byCp;
+};
+
+struct DirectExchangeArgs : DirectRanks {
   // partial_o: 16-byte units, a wavefront moves 64 consecutive ones ("chunk") of one (sender, receiver) pair
   uint32_t units;       // of one pair: entries * rowUnits
   uint32_t rowUnits;    // of one row
   FastDiv byRowUnits;
-  uint32_t waves;
   uint32_t groupShift;  // 2^groupShift consecutive wavefronts take consecutive chunks of one pair
   // softmax_stats: 8-byte pieces, all pairs together in the order (entry, receiver, sender, piece)
   uint32_t pieces;
@@ -37,7 +41,20 @@ struct DirectArgs {
   uint32_t statsBlocks;  // workgroups that move statistics; they come first in the launch
 };
 
+struct DirectCombineArgs : DirectRanks {
+  // pieces of 16 bytes (8 where head_dim is no multiple of 8): a lane makes one piece of the combined output
+  uint32_t outPieces;   // of one rank's output
+  uint32_t rowPieces;   // of a row, heads * headPieces
+  uint32_t headPieces;  // of a head
+  uint32_t heads;       // heads of a row
+  FastDiv byHeadPieces, byHeads;
+  int statsMode, lseBase2;
+};
+
 // out[r][e, s, :] = in[s][e, r, :] for both fields and all ranks of `a`.
 hipError_t launch_direct_exchange(const KernelArgs& a, const uint64_t* broken, hipStream_t stream);
+// out[r][e, h, :] = sum over s of w[s] * in[s][e, r, h, :], w = softmax over the ranks of the head's log-sum-exps
+// (patches/dcp_alltoall_helix.py:142-207); a.heads, headDim, statsMode, lseBase2 and dtype are set.
+hipError_t launch_direct_combine(const KernelArgs& a, const uint64_t* broken, hipStream_t stream);
 
 }  // namespace helix

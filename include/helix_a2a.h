@@ -233,9 +233,10 @@ int helix_a2a_alltoall_loopback(const helix_a2a_params_t* per_rank, int cp_size,
 int helix_a2a_alltoall_loopback_static(const helix_a2a_params_t* per_rank, int cp_size, int reset, void* stream);
 
 /*
- * Loopback exchange fused with the LSE-weighted combine: the receive half
- * reduces the cp_size partial outputs of each (entry, head) instead of storing
- * them. recv_fields of per_rank are ignored; out[r] receives rank r's result.
+ * Loopback exchange fused with the LSE-weighted combine: the cp_size partial
+ * outputs of each (entry, head) are reduced instead of stored, straight from the
+ * send tensors, or with a channel count (see helix_a2a_alltoall_loopback) by the
+ * receive half of the FIFO protocol. recv_fields of per_rank are ignored; out[r] receives rank r's result.
  * stats_mode is one of HELIX_A2A_STATS_*, optionally or-ed with HELIX_A2A_STATS_BASE2.
  * heads = send_fields[1].element_count / 2 (element_count itself for HELIX_A2A_STATS_LSE_PACKED),
  * head_dim = send_fields[0].element_count / heads; head_dim must be a multiple of 4 and at least 32.

@@ -93,3 +93,73 @@ def test_direct_and_fifo_exchanges_alternate_on_one_workspace(hx, ops):
         for got, ins, view in ((outs_o, ins_o, torch.int16), (outs_s, ins_s, torch.int32)):
             for r, want in enumerate(ho.exchange_single_copy([t.view(view) for t in ins])):
                 assert torch.equal(got[r].view(view), want), (i, r)
+
+
+# (cp, entries, heads per rank, head_dim, dtype, stats mode, base 2)
+COMBINE_CASES = [
+    (1, 1, 1, 32, torch.bfloat16, 1, False),     # four lanes with work
+    (4, 3, 5, 32, torch.bfloat16, 1, False),     # sixteen heads to an access, the most there can be
+    (5, 13, 3, 40, torch.float16, 0, True),      # five pieces a head: heads straddle accesses
+    (8, 7, 2, 36, torch.bfloat16, 1, False),     # 8-byte pieces, nine a head
+    (9, 5, 4, 44, torch.float16, 2, True),       # ... and a row of 8-byte pieces in groups of sixteen lanes
+    (16, 31, 1, 128, torch.bfloat16, 2, False),
+    (17, 9, 2, 64, torch.bfloat16, 1, False),    # thirty-two lanes to a head: several passes over the heads of an access
+    (32, 6, 3, 32, torch.float16, 2, False),
+    (8, 1, 1, 576, torch.bfloat16, 2, True),     # a head longer than an access
+    (8, 600, 8, 128, torch.bfloat16, 1, False),  # 79 MB of partial outputs: read past the memory-side cache
+    (4, 640, 30, 132, torch.bfloat16, 1, False), # ... in 8-byte pieces
+]
+
+
+@pytest.mark.parametrize("cp,entries,heads,d,dtype,mode,base2", COMBINE_CASES)
+def test_direct_combine(hx, ops, cp, entries, heads, d, dtype, mode, base2):
+    """Against the oracle's combine in double precision: the kernel sums at most 32 products in fp32 (2^-24 each) and
+    rounds once to the inputs' type: 8 significant bits of bf16 are off by at most 2^-8 of the value, 11 of fp16 by 2^-11; its exp, log and reciprocal are good to
+    a few ulp of fp32, times log-sum-exps of up to 20, so 2^-17 of the largest partial output covers the rest."""
+    import numpy as np
+
+    ws = workspace(hx, cp)
+    g = torch.Generator(device="cuda").manual_seed(cp * 1000 + entries)
+    ins_o = [torch.randn(entries, cp, heads * d, generator=g, device="cuda").to(dtype) for _ in range(cp)]
+    lse = [torch.randn(entries, cp, heads, generator=g, device="cuda") * 3 for _ in range(cp)]
+    for r, t in enumerate(lse):
+        t[torch.rand(t.shape, generator=g, device="cuda") < 0.1] = (float("-inf"), float("inf"), float("nan"))[r % 3]
+        t[0, :, 0] = float("-inf")  # a head that every rank masks
+    if mode == 2:
+        ins_s = lse
+    else:
+        second = torch.rand(entries, cp, heads, generator=g, device="cuda") * 50 + 1
+        ins_s = [torch.stack((t, second), -1).reshape(entries, cp, 2 * heads).contiguous() for t in lse]
+    if mode == 2:
+        # the packed form: [B, H, D] and [B, H] per rank
+        combined, glse = hx.dcp_a2a_lse_reduce([t.view(entries, cp * heads, d) for t in ins_o],
+                                               [t.view(entries, cp * heads) for t in ins_s], ws, return_lse=True,
+                                               is_lse_base_on_e=not base2)
+    else:
+        mode_bits = mode | (ops.STATS_BASE2 if base2 else 0)
+        plan = ops.CombinePlan(ins_o, ins_s, ws, mode, True)
+        plan.stats_mode = mode_bits
+        combined, glse = plan.run()
+    torch.cuda.synchronize()
+    assert ops.device_status() == 0
+    ln2 = float(np.log(2.0))
+    roundoff = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for r in range(cp):
+        o = np.stack([t[:, r].float().cpu().numpy().reshape(entries, heads, d) for t in ins_o])
+        if mode == 2:
+            l = np.stack([t[:, r].cpu().numpy() for t in ins_s]).astype(np.float64)
+        else:
+            l = ho.lse_from_stats(np.stack([t[:, r].cpu().numpy().reshape(entries, heads, 2) for t in ins_s]).astype(np.float64), mode)
+        with np.errstate(all="ignore"):
+            want, want_lse = ho.lse_combine(o, l * ln2 if base2 else l, np.float64)
+        if base2:
+            want_lse = want_lse / ln2
+        got = combined[r].float().cpu().numpy().reshape(want.shape)
+        bound = np.abs(want) * roundoff * 1.01 + np.abs(o).max() * 2.0 ** -17 + (2.0 ** -24 if dtype == torch.float16 else 0)
+        worst = float(np.max(np.abs(got - want) / bound))
+        assert worst <= 1.0, f"rank {r}: {worst} times the bound"
+        got_lse = glse[r].cpu().numpy()
+        assert np.array_equal(np.isneginf(got_lse), np.isneginf(want_lse))
+        finite = np.isfinite(want_lse)
+        worst = float(np.max(np.abs(got_lse[finite] - want_lse[finite]) / np.maximum(np.abs(want_lse[finite]), 4.0), initial=0.0))
+        assert worst <= 2.0 ** -17, f"log-sum-exp of rank {r}: {worst}"
