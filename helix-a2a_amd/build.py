@@ -1,4 +1,4 @@
-"""Build libhelix_a2a.so for gfx950 with hipcc.
+"""Build libhelix_a2a.so for gfx950 with hipcc, and the package's native module with the host compiler.
 
     python helix-a2a_amd/build.py
 
@@ -57,6 +57,35 @@ def build_library(verbose: bool = True, timeline: bool = False) -> Path:
     return output
 
 
+NATIVE_SOURCE = HERE / "csrc" / "helix_torch.cpp"
+NATIVE_OUTPUT = HERE / "helix_a2a" / "_native.so"
+
+
+def build_native_module(verbose: bool = True) -> Path:
+    """The package's native module: host code against torch's and Python's headers, no GPU code."""
+    import sysconfig
+
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+
+    rocm = Path(os.environ.get("ROCM_PATH", "/opt/rocm"))
+    includes = [*include_paths(), str(rocm / "include"), sysconfig.get_paths()["include"]]
+    libdirs = [*library_paths(), str(rocm / "lib")]
+    cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-I{d}" for d in includes), str(NATIVE_SOURCE), "-o", str(NATIVE_OUTPUT),
+           *(f"-L{d}" for d in libdirs), *(f"-Wl,-rpath,{d}" for d in library_paths()),
+           "-ltorch_python", "-ltorch_cpu", "-ltorch", "-lc10", "-lc10_hip", "-lamdhip64"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if verbose and (proc.stdout + proc.stderr).strip():
+        print(proc.stdout + proc.stderr, flush=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"{cmd[0]} failed with exit code {proc.returncode}\n{proc.stdout}{proc.stderr}")
+    return NATIVE_OUTPUT
+
+
 PROBE_SOURCE = HERE / "benchmark" / "memory_probe.hip"
 PROBE_OUTPUT = HERE / "benchmark" / "libhelix_memory_probe.so"
 
@@ -77,5 +106,6 @@ if __name__ == "__main__":
         out = build_memory_probe()
     else:
         out = build_library(timeline="--timeline" in sys.argv[1:])
+        build_native_module()
     print(f"built {out}")
     sys.exit(0)

@@ -1,0 +1,790 @@
+// helix_torch.cpp -- the tensor-level calls of the Python package in native code.
+//
+// Takes the part of the reference's libtorch binding (csrc/torch_binding.cpp:65-175): checks the tensors, allocates
+// the outputs, fills the launch descriptors of include/helix_a2a.h and makes the C call. A decode step is bound by
+// this path, not by the kernels, as long as its batch is small: at cp = 8 the same steps written in Python over
+// ctypes took 18 us per dcp_a2a_lse_reduce and 43 us per exchange of eight alltoall calls, whatever the size.
+//
+// Nothing about a tensor is kept from one call to the next. The one thing that lives between calls is a
+// LogicalRankGroup, the ranks of an exchange that have called so far.
+#define PY_SSIZE_T_CLEAN
+#include <Python.h>
+
+#include <ATen/ATen.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+#include <hip/hip_runtime_api.h>
+#include <torch/csrc/autograd/python_variable.h>
+
+#include <chrono>
+#include <cstdlib>
+#include <mutex>
+#include <stdexcept>
+#include <string>
+#include <vector>
+
+#include "../../include/helix_a2a.h"
+
+namespace {
+
+constexpr int kMaxCp = HELIX_A2A_MAX_CP_SIZE;
+
+// The entry points of the library the package has loaded (bind()).
+struct Library {
+  int (*maxChannelCount)(int, int);
+  int (*send)(const helix_a2a_params_t*, int, void*);
+  int (*recv)(const helix_a2a_params_t*, int, void*);
+  int (*loopback)(const helix_a2a_params_t*, int, void*);
+  int (*combine)(const helix_a2a_params_t*, const helix_a2a_combine_out_t*, int, int, int, void*);
+  const char* (*lastError)();
+} lib;
+
+bool g_eagerSend = false;
+double g_pendingExpiry = 120.0;
+PyObject* g_groups = nullptr;  // dict: (workspace address, cp_size) -> LogicalRankGroup
+std::mutex g_launchMutex;      // one exchange is enqueued at a time: its launches stay together on their stream
+
+struct PythonError {};  // a Python exception is set already
+
+// the reference reports user errors as RuntimeError (TORCH_CHECK)
+inline void require(bool ok, const char* message) {
+  if (!ok) throw std::runtime_error(message);
+}
+inline void require(bool ok, const std::string& message) {
+  if (!ok) throw std::runtime_error(message);
+}
+[[noreturn]] void raise_last(const char* prefix) { throw std::runtime_error(std::string(prefix) + ": " + lib.lastError()); }
+
+template <class F>
+PyObject* guarded(F&& body) {
+  try {
+    return body();
+  } catch (const PythonError&) {
+  } catch (const c10::Error& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+  } catch (const std::exception& e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+  }
+  return nullptr;
+}
+
+int as_int(PyObject* o) {
+  const long v = PyLong_AsLong(o);
+  if (v == -1 && PyErr_Occurred()) throw PythonError{};
+  require(v >= INT32_MIN && v <= INT32_MAX, "integer argument out of range");
+  return static_cast<int>(v);
+}
+
+const at::Tensor& as_tensor(PyObject* o, const char* message) {
+  require(THPVariable_Check(o), message);
+  return THPVariable_Unpack(o);
+}
+
+// A list or tuple (anything else is turned into one) of tensors.
+class TensorList {
+ public:
+  TensorList(PyObject* o, const char* message) : seq_(PySequence_Fast(o, message)) {
+    if (!seq_) throw PythonError{};
+  }
+  ~TensorList() { Py_DECREF(seq_); }
+  TensorList(const TensorList&) = delete;
+  TensorList& operator=(const TensorList&) = delete;
+  int size() const {
+    const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq_);
+    return n > kMaxCp ? kMaxCp + 1 : static_cast<int>(n);
+  }
+  const at::Tensor& at(int i) const {
+    return as_tensor(PySequence_Fast_GET_ITEM(seq_, i), "partial_o and softmax_stats must be tensors");
+  }
+
+ private:
+  PyObject* seq_;
+};
+
+void check_workspace(const at::Tensor& ws, int cp) {
+  require(ws.is_cuda(), "workspace must be on the GPU");
+  require(ws.scalar_type() == at::kLong, "workspace must be int64 (used as uint64)");
+  require(ws.dim() == 2, "workspace must be 2D (one row per rank)");
+  require(ws.size(0) == cp, "workspace must have cp_size rows");
+  require(ws.stride(1) == 1, "workspace rows must be contiguous");
+}
+
+// Entry count and row widths of a (partial_o, softmax_stats) pair.
+struct Shape {
+  int entries = 0, row0 = 0, row1 = 0;
+  bool fourD = false;  // [T, cp, H/cp, D] and [T, cp, H/cp, S], the cp axis second
+};
+
+Shape check_pair(const at::Tensor& o, const at::Tensor& s, int cp) {
+  require(o.is_cuda(), "partial_o must be on the GPU");
+  require(s.is_cuda(), "softmax_stats must be on the GPU");
+  require(o.is_contiguous(), "partial_o must be contiguous");
+  require(s.is_contiguous(), "softmax_stats must be contiguous");
+  require(o.scalar_type() == at::kHalf || o.scalar_type() == at::kBFloat16, "partial_o must be half or bfloat16");
+  require(s.scalar_type() == at::kFloat, "softmax_stats must be float32");
+  const auto os = o.sizes(), ss = s.sizes();
+  require(os.size() >= 2, "partial_o must have at least 2 dimensions");
+  require(ss.size() >= 2, "softmax_stats must have at least 2 dimensions");
+  require(os.size() == ss.size(), "partial_o and softmax_stats must have the same number of dimensions");
+  Shape shape;
+  int64_t row0 = os.back(), row1 = ss.back(), entries = 1;
+  if (os.size() == 4 && os[1] == cp && ss[1] == cp && !(os[2] == cp && ss[2] == cp)) {
+    require(os[0] == ss[0] && os[2] == ss[2], "4-D inputs must agree in their token and head dimensions");
+    shape.fourD = true;
+    entries = os[0];
+    row0 *= os[2];
+    row1 *= ss[2];
+  } else {
+    require(os[os.size() - 2] == cp && ss[ss.size() - 2] == cp, "second-to-last dimension must equal cp_size");
+    require(os.slice(0, os.size() - 2) == ss.slice(0, ss.size() - 2),
+            "partial_o and softmax_stats must have matching dimensions except the last two");
+    for (size_t i = 0; i + 2 < os.size(); ++i) entries *= os[i];
+  }
+  require(row1 >= 2 && row1 % 2 == 0, "softmax_stats last dimension must be even and >= 2");
+  require(row0 * 2 % 16 == 0, "partial_o rows must be a multiple of 16 bytes");
+  require(entries <= INT32_MAX && row0 <= INT32_MAX / 2 && row1 <= INT32_MAX / 4, "partial_o and softmax_stats are too large");
+  shape.entries = static_cast<int>(entries);
+  shape.row0 = static_cast<int>(row0);
+  shape.row1 = static_cast<int>(row1);
+  return shape;
+}
+
+bool same_pair(const at::Tensor& o, const at::Tensor& s, const at::Tensor& o0, const at::Tensor& s0) {
+  return o.sizes() == o0.sizes() && s.sizes() == s0.sizes() && o.scalar_type() == o0.scalar_type() &&
+         s.scalar_type() == s0.scalar_type();
+}
+
+helix_a2a_field_t field(const void* data, int count, int size) {
+  helix_a2a_field_t f;
+  f.data = const_cast<void*>(data);
+  f.element_count = count;
+  f.element_size = size;
+  f.stride_bytes = count * size;
+  return f;
+}
+
+// The descriptor of rank `rank`; data pointers of the outputs are null where the call has none.
+void fill_params(helix_a2a_params_t& p, int rank, int cp, int entries, const at::Tensor& o, const at::Tensor& s, void* outO,
+                 void* outS, int row0, int row1, const at::Tensor& ws, int channels, int maxChannels) {
+  p.send_fields[0] = field(o.const_data_ptr(), row0, 2);
+  p.send_fields[1] = field(s.const_data_ptr(), row1, 4);
+  p.recv_fields[0] = field(outO, row0, 2);
+  p.recv_fields[1] = field(outS, row1, 4);
+  p.entry_count = entries;
+  p.workspace = static_cast<uint64_t*>(ws.data_ptr());
+  p.workspace_stride_u64 = static_cast<uint64_t>(ws.stride(0));
+  p.cp_rank = rank;
+  p.cp_size = cp;
+  p.channel_count = channels;
+  p.max_channel_count = maxChannels;
+}
+
+int device_max_channels(int cp) {
+  const int n = lib.maxChannelCount(cp, 0);
+  if (n < 0) raise_last("max_channel_count");
+  return n;
+}
+
+// One allocation for the outputs of all ranks, rank r's is slice r.
+struct Outputs {
+  at::Tensor all;
+  std::vector<int64_t> sizes;  // of a slice
+  int64_t numel = 1;
+  Outputs() = default;
+  Outputs(int cp, at::IntArrayRef slice, at::ScalarType dtype, const at::Device& device) : sizes(slice.vec()) {
+    std::vector<int64_t> full;
+    full.reserve(slice.size() + 1);
+    full.push_back(cp);
+    for (int64_t d : slice) {
+      full.push_back(d);
+      numel *= d;
+    }
+    all = at::empty(full, at::TensorOptions().dtype(dtype).device(device));
+  }
+  at::Tensor slice(int r) const {
+    at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(all.storage()), all.key_set(), all.dtype());
+    t.unsafeGetTensorImpl()->set_storage_offset(r * numel);
+    t.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+    return t;
+  }
+  void* data(int r) const { return static_cast<char*>(all.data_ptr()) + r * numel * static_cast<int64_t>(all.element_size()); }
+};
+
+PyObject* wrap_slices(const Outputs& out, int cp) {
+  PyObject* list = PyList_New(cp);
+  if (!list) throw PythonError{};
+  for (int r = 0; r < cp; ++r) {
+    PyObject* t = THPVariable_Wrap(out.slice(r));
+    if (!t) {
+      Py_DECREF(list);
+      throw PythonError{};
+    }
+    PyList_SET_ITEM(list, r, t);
+  }
+  return list;
+}
+
+PyObject* pair(PyObject* a, PyObject* b) {
+  PyObject* t = PyTuple_New(2);
+  if (!t) {
+    Py_DECREF(a);
+    Py_DECREF(b);
+    throw PythonError{};
+  }
+  PyTuple_SET_ITEM(t, 0, a);
+  PyTuple_SET_ITEM(t, 1, b);
+  return t;
+}
+
+// The C call, without the interpreter lock: in checked mode it waits for the stream.
+template <class F>
+void launch(const char* what, F&& call) {
+  int rc;
+  Py_BEGIN_ALLOW_THREADS
+  {
+    std::lock_guard<std::mutex> lock(g_launchMutex);
+    rc = call();
+  }
+  Py_END_ALLOW_THREADS
+  if (rc != 0) raise_last(what);
+}
+
+hipStream_t current_stream(const at::Device& device) { return c10::hip::getCurrentHIPStream(device.index()).stream(); }
+
+// ---------------------------------------------------------------------------
+// all ranks in one call
+// ---------------------------------------------------------------------------
+
+// alltoall_loopback(partial_o, softmax_stats, workspace, channel_count, out)
+PyObject* alltoall_loopback(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    require(nargs == 5, "alltoall_loopback takes 5 arguments");
+    const TensorList os(args[0], "partial_o must be a sequence"), ss(args[1], "softmax_stats must be a sequence");
+    const int cp = os.size();
+    require(cp >= 1 && cp <= kMaxCp && ss.size() == cp, "need one partial_o and one softmax_stats tensor per rank");
+    const at::Tensor& ws = as_tensor(args[2], "workspace must be on the GPU");
+    check_workspace(ws, cp);
+    const int channels = as_int(args[3]);
+    const at::Tensor &o0 = os.at(0), &s0 = ss.at(0);
+    const Shape shape = check_pair(o0, s0, cp);
+    const at::Device device = ws.device();
+    const c10::DeviceGuard guard(device);
+
+    Outputs outO, outS;
+    PyObject *givenO = nullptr, *givenS = nullptr;
+    if (args[4] == Py_None) {
+      outO = Outputs(cp, o0.sizes(), o0.scalar_type(), device);
+      outS = Outputs(cp, s0.sizes(), at::kFloat, device);
+    } else {
+      PyObject* seq = PySequence_Fast(args[4], "out must be a pair of sequences");
+      if (!seq) throw PythonError{};
+      const bool two = PySequence_Fast_GET_SIZE(seq) == 2;
+      givenO = two ? PySequence_List(PySequence_Fast_GET_ITEM(seq, 0)) : nullptr;
+      givenS = two && givenO ? PySequence_List(PySequence_Fast_GET_ITEM(seq, 1)) : nullptr;
+      Py_DECREF(seq);
+      if (!givenS) {
+        Py_XDECREF(givenO);
+        if (PyErr_Occurred()) throw PythonError{};
+        throw std::runtime_error("need one output pair per rank");
+      }
+    }
+    try {
+      require(!givenO || (PyList_GET_SIZE(givenO) == cp && PyList_GET_SIZE(givenS) == cp), "need one output pair per rank");
+      helix_a2a_params_t params[kMaxCp];
+      const int maxChannels = device_max_channels(cp);
+      for (int r = 0; r < cp; ++r) {
+        const at::Tensor &o = os.at(r), &s = ss.at(r);
+        if (r > 0) {
+          require(o.is_cuda(), "partial_o must be on the GPU");
+          require(s.is_cuda(), "softmax_stats must be on the GPU");
+          require(same_pair(o, s, o0, s0), "all ranks must exchange tensors of one shape and dtype");
+          require(o.is_contiguous(), "partial_o must be contiguous");
+          require(s.is_contiguous(), "softmax_stats must be contiguous");
+        }
+        require(o.device() == device && s.device() == device, "all tensors must live on one device");
+        void *po, *ps;
+        if (givenO) {
+          const at::Tensor& oo = as_tensor(PyList_GET_ITEM(givenO, r), "out tensors must match the inputs");
+          const at::Tensor& so = as_tensor(PyList_GET_ITEM(givenS, r), "out tensors must match the inputs");
+          require(same_pair(oo, so, o, s) && oo.is_contiguous() && so.is_contiguous() && oo.is_cuda() && so.is_cuda(),
+                  "out tensors must match the inputs");
+          po = oo.data_ptr();
+          ps = so.data_ptr();
+        } else {
+          po = outO.data(r);
+          ps = outS.data(r);
+        }
+        fill_params(params[r], r, cp, shape.entries, o, s, po, ps, shape.row0, shape.row1, ws, channels, maxChannels);
+      }
+      const hipStream_t stream = current_stream(device);
+      launch("alltoall_loopback", [&] { return lib.loopback(params, cp, stream); });
+    } catch (...) {
+      Py_XDECREF(givenO);
+      Py_XDECREF(givenS);
+      throw;
+    }
+    if (givenO) return pair(givenO, givenS);
+    PyObject* first = wrap_slices(outO, cp);
+    return pair(first, wrap_slices(outS, cp));
+  });
+}
+
+// The combined outputs of all ranks (and their log-sum-exps) as Python lists.
+PyObject* combine_result(const Outputs& combined, const Outputs& lse, int cp, bool returnLse) {
+  PyObject* first = wrap_slices(combined, cp);
+  return returnLse ? pair(first, wrap_slices(lse, cp)) : first;
+}
+
+// alltoall_combine_loopback(partial_o, softmax_stats, workspace, stats_mode, return_lse, channel_count)
+PyObject* alltoall_combine_loopback(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    require(nargs == 6, "alltoall_combine_loopback takes 6 arguments");
+    const TensorList os(args[0], "partial_o must be a sequence"), ss(args[1], "softmax_stats must be a sequence");
+    const int cp = os.size();
+    require(cp >= 1 && cp <= HELIX_A2A_MAX_COMBINE_CP_SIZE && ss.size() == cp,
+            "need one partial_o and one softmax_stats tensor per rank, at most 32 ranks");
+    const int mode = as_int(args[3]);
+    require(mode == HELIX_A2A_STATS_LSE || mode == HELIX_A2A_STATS_MAX_SUM || mode == HELIX_A2A_STATS_LSE_PACKED,
+            "stats_mode must be STATS_LSE, STATS_MAX_SUM or STATS_LSE_PACKED");
+    const int returnLse = PyObject_IsTrue(args[4]);
+    if (returnLse < 0) throw PythonError{};
+    const at::Tensor& ws = as_tensor(args[2], "workspace must be on the GPU");
+    check_workspace(ws, cp);
+    const int channels = as_int(args[5]);
+    const at::Tensor &o0 = os.at(0), &s0 = ss.at(0);
+    const Shape shape = check_pair(o0, s0, cp);
+    const int heads = mode == HELIX_A2A_STATS_LSE_PACKED ? shape.row1 : shape.row1 / 2;
+    require(shape.row0 % heads == 0 && (shape.row0 / heads) % 4 == 0 && shape.row0 / heads >= 32,
+            "partial_o rows must hold heads * head_dim elements, head_dim a multiple of 4 and >= 32");
+    const at::Device device = ws.device();
+    const c10::DeviceGuard guard(device);
+
+    Outputs combined, lse;
+    if (o0.dim() == 4 && o0.size(1) == cp && o0.size(2) == heads)
+      combined = Outputs(cp, {shape.entries, heads, shape.row0 / heads}, o0.scalar_type(), device);
+    else
+      combined = Outputs(cp, {shape.entries, shape.row0}, o0.scalar_type(), device);
+    if (returnLse) lse = Outputs(cp, {shape.entries, heads}, at::kFloat, device);
+    helix_a2a_params_t params[kMaxCp];
+    helix_a2a_combine_out_t out[kMaxCp];
+    const int maxChannels = device_max_channels(cp);
+    for (int r = 0; r < cp; ++r) {
+      const at::Tensor &o = os.at(r), &s = ss.at(r);
+      if (r > 0) {
+        require(o.is_cuda(), "partial_o must be on the GPU");
+        require(s.is_cuda(), "softmax_stats must be on the GPU");
+        require(same_pair(o, s, o0, s0), "all ranks must exchange tensors of one shape and dtype");
+        require(o.is_contiguous(), "partial_o must be contiguous");
+        require(s.is_contiguous(), "softmax_stats must be contiguous");
+      }
+      require(o.device() == device && s.device() == device, "all tensors must live on one device");
+      fill_params(params[r], r, cp, shape.entries, o, s, nullptr, nullptr, shape.row0, shape.row1, ws, channels, maxChannels);
+      out[r].combined = combined.data(r);
+      out[r].lse_out = returnLse ? static_cast<float*>(lse.data(r)) : nullptr;
+    }
+    const hipStream_t stream = current_stream(device);
+    const int dtype = o0.scalar_type() == at::kBFloat16 ? HELIX_A2A_DTYPE_BF16 : HELIX_A2A_DTYPE_FP16;
+    launch("alltoall_combine_loopback", [&] { return lib.combine(params, out, cp, mode, dtype, stream); });
+    return combine_result(combined, lse, cp, returnLse != 0);
+  });
+}
+
+// dcp_reduce(cp_attn_out, cp_attn_lse, workspace, return_lse, channel_count, lse_base2)
+PyObject* dcp_reduce(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    require(nargs == 6, "dcp_reduce takes 6 arguments");
+    const TensorList os(args[0], "cp_attn_out must be a sequence"), ls(args[1], "cp_attn_lse must be a sequence");
+    const int n = os.size();
+    require(n >= 1 && n <= HELIX_A2A_MAX_COMBINE_CP_SIZE && ls.size() == n,
+            "need one attention output and one LSE tensor per rank, at most 32 ranks");
+    const at::Tensor& o0 = os.at(0);
+    require(o0.dim() == 3, "expected cp_attn_out [B, H, D]");
+    const int64_t b = o0.size(0), h = o0.size(1), d = o0.size(2);
+    require(o0.scalar_type() == at::kHalf || o0.scalar_type() == at::kBFloat16, "cp_attn_out must be half or bfloat16");
+    require(o0.is_cuda(), "cp_attn_out must be on the GPU");
+    require(h % n == 0, "H must be divisible by the rank count");
+    const int64_t hp = h / n;
+    require(d % 4 == 0 && d >= 32, "head_dim must be a multiple of 4 and >= 32");
+    const at::Tensor& ws = as_tensor(args[2], "workspace must be on the GPU");
+    check_workspace(ws, n);
+    const at::Device device = o0.device();
+    require(ws.device() == device, "all tensors must live on one device");
+    require(b <= INT32_MAX && hp * d <= INT32_MAX / 2, "cp_attn_out is too large");
+    const int returnLse = PyObject_IsTrue(args[3]), base2 = PyObject_IsTrue(args[5]);
+    if (returnLse < 0 || base2 < 0) throw PythonError{};
+    const int channels = as_int(args[4]);
+    const c10::DeviceGuard guard(device);
+
+    Outputs combined(n, {b, hp, d}, o0.scalar_type(), device), lse;
+    if (returnLse) lse = Outputs(n, {b, hp}, at::kFloat, device);
+    std::vector<at::Tensor> keep;  // contiguous copies, until the launch is enqueued
+    helix_a2a_params_t params[kMaxCp];
+    helix_a2a_combine_out_t out[kMaxCp];
+    const int maxChannels = device_max_channels(n);
+    const int64_t lseSizes[2] = {b, h};
+    for (int r = 0; r < n; ++r) {
+      const at::Tensor *o = &os.at(r), *l = &ls.at(r);
+      require(o->sizes() == o0.sizes() && o->scalar_type() == o0.scalar_type() && o->device() == device,
+              "all ranks must pass cp_attn_out of one shape, dtype and device");
+      require(l->sizes() == at::IntArrayRef(lseSizes, 2) && l->scalar_type() == at::kFloat && l->device() == device,
+              "cp_attn_lse must be float32 [B, H] on the same device");
+      if (!o->is_contiguous() || !l->is_contiguous()) {
+        if (keep.empty()) keep.reserve(2 * kMaxCp);
+        keep.push_back(o->contiguous());
+        o = &keep.back();
+        keep.push_back(l->contiguous());
+        l = &keep.back();
+      }
+      fill_params(params[r], r, n, static_cast<int>(b), *o, *l, nullptr, nullptr, static_cast<int>(hp * d), static_cast<int>(hp), ws,
+                  channels, maxChannels);
+      out[r].combined = combined.data(r);
+      out[r].lse_out = returnLse ? static_cast<float*>(lse.data(r)) : nullptr;
+    }
+    const hipStream_t stream = current_stream(device);
+    const int dtype = o0.scalar_type() == at::kBFloat16 ? HELIX_A2A_DTYPE_BF16 : HELIX_A2A_DTYPE_FP16;
+    const int mode = HELIX_A2A_STATS_LSE_PACKED | (base2 ? HELIX_A2A_STATS_BASE2 : 0);
+    launch("dcp_a2a_lse_reduce", [&] { return lib.combine(params, out, n, mode, dtype, stream); });
+    return combine_result(combined, lse, n, returnLse != 0);
+  });
+}
+
+// run_loopback(address of the descriptors, cp_size), run_combine(descriptors, outputs, cp_size, stats_mode, dtype): the
+// call of a plan, whose descriptors are filled once, on the current stream of the current device.
+PyObject* run_loopback(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    require(nargs == 2, "run_loopback takes 2 arguments");
+    const auto* params = static_cast<const helix_a2a_params_t*>(PyLong_AsVoidPtr(args[0]));
+    const int cp = as_int(args[1]);
+    const hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
+    launch("alltoall_loopback", [&] { return lib.loopback(params, cp, stream); });
+    Py_RETURN_NONE;
+  });
+}
+PyObject* run_combine(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    require(nargs == 5, "run_combine takes 5 arguments");
+    const auto* params = static_cast<const helix_a2a_params_t*>(PyLong_AsVoidPtr(args[0]));
+    const auto* out = static_cast<const helix_a2a_combine_out_t*>(PyLong_AsVoidPtr(args[1]));
+    const int cp = as_int(args[2]), mode = as_int(args[3]), dtype = as_int(args[4]);
+    const hipStream_t stream = c10::hip::getCurrentHIPStream().stream();
+    launch("alltoall_combine_loopback", [&] { return lib.combine(params, out, cp, mode, dtype, stream); });
+    Py_RETURN_NONE;
+  });
+}
+
+// ---------------------------------------------------------------------------
+// one call per rank
+// ---------------------------------------------------------------------------
+
+double now_seconds() {
+  return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
+}
+
+// HELIX_A2A_CHANNEL_COUNT (csrc/torch_binding.cpp:25-32), 0 when unset or not a positive number.
+int env_channel_count() {
+  const char* env = std::getenv("HELIX_A2A_CHANNEL_COUNT");
+  if (!env || !*env) return 0;
+  char* end = nullptr;
+  const long n = std::strtol(env, &end, 10);
+  while (end && (*end == ' ' || *end == '\n' || *end == '\t')) ++end;
+  return end && *end == '\0' && n > 0 && n <= INT32_MAX ? static_cast<int>(n) : 0;
+}
+
+// What the ranks of an exchange that have called so far left behind.
+struct Exchange {
+  uint32_t called = 0;  // bit r: rank r
+  int calls = 0;
+  int channels = 0, maxChannels = 0;
+  bool eager = false;
+  double started = 0.0;
+  Shape shape;
+  at::Tensor workspace;  // kept while ranks are pending: the caller may have passed a temporary view
+  at::Tensor o[kMaxCp], s[kMaxCp];
+  Outputs outO, outS;
+  hipStream_t stream[kMaxCp];
+  helix_a2a_params_t params[kMaxCp];
+};
+
+// The ranks of one workspace that share this device.
+//
+// A rank's receive half depends on every peer's send half, so nothing can complete before the last rank of the group
+// has called. By default the whole exchange is therefore issued by that call, as one launch of all ranks on the last
+// caller's stream; until then the group keeps the ranks' tensors (and the workspace) alive, and a rank must leave its
+// inputs alone. With eager sends a rank's call enqueues its send half at once and only the receive halves wait for
+// the last rank -- unless the exchange is too large for the four FIFO entries of a stream (a send launch cannot be
+// back-pressured by a receive launch queued behind it), which falls back to the one launch.
+//
+// The outputs of all ranks are two allocations made by the first rank's call; every rank is handed its slice.
+//
+// The channel count of an exchange (HELIX_A2A_CHANNEL_COUNT or automatic) is settled by its first rank's call and
+// used for every launch of it, whatever the environment says later.
+struct Group {
+  PyObject_HEAD
+  int cp;
+  Exchange* ex;  // null between exchanges
+};
+
+void group_dealloc(PyObject* self) {
+  delete reinterpret_cast<Group*>(self)->ex;
+  Py_TYPE(self)->tp_free(self);
+}
+
+std::string rank_list(uint32_t mask) {
+  std::string s = "[";
+  for (int r = 0; r < kMaxCp; ++r)
+    if (mask & (1u << r)) s += (s.size() > 1 ? ", " : "") + std::to_string(r);
+  return s + "]";
+}
+
+PyObject* group_pending(PyObject* self, void*) {
+  const Exchange* ex = reinterpret_cast<Group*>(self)->ex;
+  PyObject* list = PyList_New(0);
+  for (int r = 0; list && ex && r < kMaxCp; ++r)
+    if (ex->called & (1u << r)) {
+      PyObject* v = PyLong_FromLong(r);
+      if (!v || PyList_Append(list, v) != 0) Py_CLEAR(list);
+      Py_XDECREF(v);
+    }
+  return list;
+}
+
+PyObject* group_workspace(PyObject* self, void*) {
+  const Exchange* ex = reinterpret_cast<Group*>(self)->ex;
+  if (!ex) Py_RETURN_NONE;
+  return THPVariable_Wrap(ex->workspace);
+}
+
+PyGetSetDef group_getset[] = {
+    {"pending", group_pending, nullptr, "ranks that have called and wait for the others", nullptr},
+    {"workspace", group_workspace, nullptr, "the workspace while ranks are pending, else None", nullptr},
+    {nullptr, nullptr, nullptr, nullptr, nullptr},
+};
+
+PyTypeObject GroupType = {PyVarObject_HEAD_INIT(nullptr, 0)};
+
+struct Event {
+  hipEvent_t handle = nullptr;
+  Event() { require(hipEventCreateWithFlags(&handle, hipEventDisableTiming) == hipSuccess, "alltoall: cannot create an event"); }
+  ~Event() { (void)hipEventDestroy(handle); }
+  Event(const Event&) = delete;
+  Event& operator=(const Event&) = delete;
+  void record(hipStream_t s) { require(hipEventRecord(handle, s) == hipSuccess, "alltoall: cannot record an event"); }
+  void hold(hipStream_t s) { require(hipStreamWaitEvent(s, handle, 0) == hipSuccess, "alltoall: cannot wait for an event"); }
+};
+
+// Enqueue what is left of the exchange on the last caller's stream. That stream first waits for the work of every
+// other stream a rank called on (its send half, or the producer of its inputs); afterwards those streams wait for
+// this launch, so each rank's outputs are valid once the stream *it* called on has drained.
+void flush(Exchange& ex, int cp, hipStream_t stream) {
+  std::vector<hipStream_t> others;
+  for (int r = 0; r < cp; ++r) {
+    const hipStream_t s = ex.stream[r];
+    bool seen = s == stream;
+    for (hipStream_t o : others) seen = seen || o == s;
+    if (!seen) others.push_back(s);
+  }
+  for (hipStream_t o : others) {
+    Event ev;
+    ev.record(o);
+    ev.hold(stream);
+  }
+  if (ex.eager)
+    launch("alltoall (receive half)", [&] { return lib.recv(ex.params, cp, stream); });
+  else
+    launch("alltoall", [&] { return lib.loopback(ex.params, cp, stream); });
+  if (!others.empty()) {
+    Event done;
+    done.record(stream);
+    for (hipStream_t o : others) done.hold(o);
+  }
+}
+
+Group* group_of(const at::Tensor& ws, int cp) {
+  PyObject* key = Py_BuildValue("(Ki)", reinterpret_cast<unsigned long long>(ws.const_data_ptr()), cp);
+  if (!key) throw PythonError{};
+  PyObject* found = PyDict_GetItemWithError(g_groups, key);
+  if (!found) {
+    bool ok = !PyErr_Occurred();
+    if (ok && PyDict_GET_SIZE(g_groups) >= 64) {  // groups between exchanges hold nothing worth keeping
+      PyObject* items = PyDict_Items(g_groups);
+      ok = items != nullptr;
+      for (Py_ssize_t i = 0; ok && i < PyList_GET_SIZE(items); ++i) {
+        PyObject* item = PyList_GET_ITEM(items, i);
+        if (!reinterpret_cast<Group*>(PyTuple_GET_ITEM(item, 1))->ex) ok = PyDict_DelItem(g_groups, PyTuple_GET_ITEM(item, 0)) == 0;
+      }
+      Py_XDECREF(items);
+    }
+    Group* group = ok ? PyObject_New(Group, &GroupType) : nullptr;
+    if (group) {
+      group->cp = cp;
+      group->ex = nullptr;
+      found = reinterpret_cast<PyObject*>(group);
+      if (PyDict_SetItem(g_groups, key, found) != 0) found = nullptr;
+      Py_DECREF(group);
+    }
+  }
+  Py_DECREF(key);
+  if (!found) throw PythonError{};
+  return reinterpret_cast<Group*>(found);
+}
+
+// alltoall(partial_o, softmax_stats, workspace, cp_rank, cp_size)
+PyObject* alltoall(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  return guarded([&]() -> PyObject* {
+    require(nargs == 5, "alltoall takes 5 arguments");
+    const int rank = as_int(args[3]), cp = as_int(args[4]);
+    require(cp >= 1 && cp <= kMaxCp, "cp_size must be in [1, 32]");
+    const at::Tensor& o = as_tensor(args[0], "partial_o and softmax_stats must be tensors");
+    const at::Tensor& s = as_tensor(args[1], "partial_o and softmax_stats must be tensors");
+    const Shape shape = check_pair(o, s, cp);
+    const at::Tensor& ws = as_tensor(args[2], "workspace must be on the GPU");
+    check_workspace(ws, cp);
+    require(rank >= 0 && rank < cp, "cp_rank must be in [0, cp_size)");
+    const at::Device device = ws.device();
+    require(device == o.device() && device == s.device(), "all tensors must live on one device");
+    const c10::DeviceGuard guard(device);
+
+    Group* group = group_of(ws, cp);
+    Exchange* ex = group->ex;
+    if (ex) {
+      if (now_seconds() - ex->started > g_pendingExpiry) {
+        const std::string waited = rank_list(ex->called);
+        group->ex = nullptr;
+        delete ex;
+        throw std::runtime_error("logical ranks " + waited + " waited more than " + std::to_string(static_cast<long>(g_pendingExpiry)) +
+                                 " s for the other ranks of their exchange; it is given up: re-initialise the workspace before the "
+                                 "next exchange");
+      }
+      require(!(ex->called & (1u << rank)), "logical rank " + std::to_string(rank) + " called alltoall again before all " +
+                                                std::to_string(cp) + " ranks of the group had called");
+      int peer = 0;
+      while (!(ex->called & (1u << peer))) ++peer;
+      require(same_pair(o, s, ex->o[peer], ex->s[peer]), "logical ranks of one group must exchange tensors of one shape and dtype");
+    } else {
+      std::unique_ptr<Exchange> fresh(new Exchange);
+      fresh->channels = env_channel_count();
+      fresh->maxChannels = device_max_channels(cp);
+      require(fresh->channels <= fresh->maxChannels, "alltoall: channel_count " + std::to_string(fresh->channels) +
+                                                         " exceeds max_channel_count " + std::to_string(fresh->maxChannels));
+      fresh->shape = shape;
+      fresh->eager = g_eagerSend;
+      fresh->started = now_seconds();
+      fresh->workspace = ws;
+      fresh->outO = Outputs(cp, o.sizes(), o.scalar_type(), device);
+      fresh->outS = Outputs(cp, s.sizes(), at::kFloat, device);
+      ex = fresh.release();
+    }
+    // from here on `ex` belongs to the group, or goes with this call
+    struct Owner {
+      Group* group;
+      Exchange* ex;
+      ~Owner() {
+        if (group->ex != ex) delete ex;
+        Py_DECREF(group);
+      }
+    } owner{group, ex};
+    Py_INCREF(group);  // the dict may let go of it while the interpreter lock is released below
+    const bool first = ex->calls == 0;
+    fill_params(ex->params[rank], rank, cp, shape.entries, o, s, ex->outO.data(rank), ex->outS.data(rank), shape.row0, shape.row1,
+                ex->workspace, ex->channels, ex->maxChannels);
+    const hipStream_t stream = current_stream(device);
+    if (ex->eager) {
+      int rc;
+      {
+        std::lock_guard<std::mutex> lock(g_launchMutex);
+        rc = lib.send(&ex->params[rank], 1, stream);
+      }
+      if (rc == HELIX_A2A_ERR_CAPACITY && first)
+        ex->eager = false;  // on the first rank: the one launch of all ranks instead
+      else if (rc != 0)
+        raise_last("alltoall (send half)");
+    }
+    ex->o[rank] = o;
+    ex->s[rank] = s;
+    ex->stream[rank] = stream;
+    ex->called |= 1u << rank;
+    ex->calls += 1;
+    PyObject* outO = THPVariable_Wrap(ex->outO.slice(rank));
+    if (!outO) throw PythonError{};
+    PyObject* outS = THPVariable_Wrap(ex->outS.slice(rank));
+    if (!outS) {
+      Py_DECREF(outO);
+      throw PythonError{};
+    }
+    PyObject* result = pair(outO, outS);
+    if (ex->calls < cp) {
+      group->ex = ex;
+      return result;
+    }
+    group->ex = nullptr;  // the next exchange may start while this one is being enqueued
+    try {
+      flush(*ex, cp, stream);
+    } catch (...) {
+      Py_DECREF(result);
+      throw;
+    }
+    return result;
+  });
+}
+
+// ---------------------------------------------------------------------------
+
+PyObject* set_eager_send(PyObject*, PyObject* arg) {
+  const int v = PyObject_IsTrue(arg);
+  if (v < 0) return nullptr;
+  g_eagerSend = v != 0;
+  Py_RETURN_NONE;
+}
+
+PyObject* set_pending_expiry(PyObject*, PyObject* arg) {
+  const double v = PyFloat_AsDouble(arg);
+  if (v == -1.0 && PyErr_Occurred()) return nullptr;
+  g_pendingExpiry = v;
+  Py_RETURN_NONE;
+}
+
+// bind(groups, addresses): the dict of logical-rank groups, and the addresses of the C entry points
+PyObject* bind(PyObject*, PyObject* args) {
+  PyObject* groups;
+  unsigned long long f[6];
+  if (!PyArg_ParseTuple(args, "O!KKKKKK", &PyDict_Type, &groups, &f[0], &f[1], &f[2], &f[3], &f[4], &f[5])) return nullptr;
+  Py_INCREF(groups);
+  Py_XSETREF(g_groups, groups);
+  lib.maxChannelCount = reinterpret_cast<decltype(lib.maxChannelCount)>(f[0]);
+  lib.send = reinterpret_cast<decltype(lib.send)>(f[1]);
+  lib.recv = reinterpret_cast<decltype(lib.recv)>(f[2]);
+  lib.loopback = reinterpret_cast<decltype(lib.loopback)>(f[3]);
+  lib.combine = reinterpret_cast<decltype(lib.combine)>(f[4]);
+  lib.lastError = reinterpret_cast<decltype(lib.lastError)>(f[5]);
+  Py_RETURN_NONE;
+}
+
+PyCFunction fast(_PyCFunctionFast f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)); }
+
+PyMethodDef methods[] = {
+    {"bind", bind, METH_VARARGS, nullptr},
+    {"alltoall", fast(alltoall), METH_FASTCALL, nullptr},
+    {"alltoall_loopback", fast(alltoall_loopback), METH_FASTCALL, nullptr},
+    {"alltoall_combine_loopback", fast(alltoall_combine_loopback), METH_FASTCALL, nullptr},
+    {"dcp_reduce", fast(dcp_reduce), METH_FASTCALL, nullptr},
+    {"run_loopback", fast(run_loopback), METH_FASTCALL, nullptr},
+    {"run_combine", fast(run_combine), METH_FASTCALL, nullptr},
+    {"set_eager_send", set_eager_send, METH_O, nullptr},
+    {"set_pending_expiry", set_pending_expiry, METH_O, nullptr},
+    {nullptr, nullptr, 0, nullptr},
+};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "helix_a2a._native", "tensor-level calls of helix_a2a", -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__native(void) {
+  GroupType.tp_name = "helix_a2a._native.LogicalRankGroup";
+  GroupType.tp_basicsize = sizeof(Group);
+  GroupType.tp_dealloc = group_dealloc;
+  GroupType.tp_flags = Py_TPFLAGS_DEFAULT;
+  GroupType.tp_getset = group_getset;
+  GroupType.tp_doc = "the logical ranks of one workspace";
+  if (PyType_Ready(&GroupType) < 0) return nullptr;
+  return PyModule_Create(&module);
+}

@@ -27,6 +27,10 @@ import torch
 
 from helix_a2a import _ops
 from helix_a2a._ops import STATS_LSE, STATS_LSE_PACKED, STATS_MAX_SUM  # noqa: F401
+from helix_a2a._native import alltoall as _alltoall
+from helix_a2a._native import alltoall_combine_loopback as _alltoall_combine_loopback
+from helix_a2a._native import alltoall_loopback as _alltoall_loopback
+from helix_a2a._native import dcp_reduce as _dcp_reduce
 from helix_a2a._version import __version__  # noqa: F401
 
 __all__ = [
@@ -104,7 +108,7 @@ def alltoall(
     returned tensors are filled once every rank has called (see the module
     docstring for what that asks of the inputs).
     """
-    return _ops.alltoall_native(partial_o, softmax_stats, workspace, cp_rank, cp_size)
+    return _alltoall(partial_o, softmax_stats, workspace, cp_rank, cp_size)
 
 
 def alltoall_loopback(
@@ -115,7 +119,7 @@ def alltoall_loopback(
     out: Optional[Tuple[Sequence[torch.Tensor], Sequence[torch.Tensor]]] = None,
 ) -> Tuple[List[torch.Tensor], List[torch.Tensor]]:
     """Exchange of all logical ranks in one launch: element ``r`` of each list is rank ``r``."""
-    return _ops.alltoall_loopback(partial_o, softmax_stats, workspace, channel_count, out)
+    return _alltoall_loopback(partial_o, softmax_stats, workspace, channel_count, out)
 
 
 def alltoall_combine_loopback(
@@ -135,7 +139,7 @@ def alltoall_combine_loopback(
     max, running sum) or ``STATS_LSE_PACKED`` (``softmax_stats`` is
     ``[..., cp_size, heads]`` with one natural-log LSE per head).
     """
-    return _ops.alltoall_combine_loopback(partial_o, softmax_stats, workspace, stats_mode, return_lse, channel_count)
+    return _alltoall_combine_loopback(partial_o, softmax_stats, workspace, stats_mode, return_lse, channel_count)
 
 
 def dcp_a2a_lse_reduce(
@@ -165,4 +169,4 @@ def dcp_a2a_lse_reduce(
     directly (the reference path permutes before and after its kernel,
     patches/dcp_alltoall_helix.py:545-593).
     """
-    return _ops.dcp_reduce(cp_attn_out, cp_attn_lse, workspace, return_lse, channel_count, lse_base2=not is_lse_base_on_e)
+    return _dcp_reduce(cp_attn_out, cp_attn_lse, workspace, return_lse, channel_count, not is_lse_base_on_e)
