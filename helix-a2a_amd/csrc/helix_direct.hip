@@ -20,31 +20,29 @@ constexpr int kAuxNtSc1 = 18;
 constexpr uint32_t kRsrcWord3 = 0x00020000u;   // raw buffer, 32-bit data format
 constexpr uint32_t kOutOfRange = 0x80000000u;  // beyond any descriptor (extents are < 2 GiB): how a lane opts out
 constexpr uint32_t kStatusBrokenWorkspace = 8u;
-constexpr int kBlockWaves = 4;
-constexpr int kBlockThreads = kBlockWaves * kWaveLanes;
 
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, static_cast<int>(bytes), kRsrcWord3);
 }
 
 // Whether the workspace was broken before this launch, read through the scalar cache (empty at every launch).
-__device__ __forceinline__ bool broken_at_launch(const DirectRanks& a) {
+__device__ __forceinline__ bool broken_at_launch(const DirectCommon& a) {
   using ConstWord = const __attribute__((address_space(4))) uint64_t;
   return *reinterpret_cast<ConstWord*>(reinterpret_cast<uintptr_t>(a.broken)) != 0;
 }
-__device__ __forceinline__ void report_broken(const DirectRanks& a) {
+__device__ __forceinline__ void report_broken(const DirectCommon& a) {
   if (threadIdx.x % kWaveLanes == 0) atomicOr(a.status, kStatusBrokenWorkspace);
 }
 
 using GlobalPiece = __attribute__((address_space(1))) u32x2;
 
-// One workgroup moves kPerThread * 256 consecutive statistics pieces in the order (entry, receiver, sender,
+// One workgroup moves kPerThread consecutive statistics pieces a thread in the order (entry, receiver, sender,
 // piece). A statistics row can be as small as 8 bytes and its neighbours go to other ranks, so the pairs are not
 // kept apart here as they are for partial_o: with all ranks in one workgroup the lines that rows of different
 // pairs share are fetched by one L2 and written from one L2, and every store covers cp consecutive rows of the
 // receiver. The rank is a lane's own then; the 2 * cp pointers go through LDS.
-template <int kPerThread>
-__device__ __forceinline__ void move_statistics(const DirectExchangeArgs& a, uint64_t (&from)[kMaxCpSize], uint64_t (&to)[kMaxCpSize]) {
+template <int kRanks, int kThreads, int kPerThread>
+__device__ __forceinline__ void move_statistics(const DirectExchangeArgs<kRanks>& a, uint64_t (&from)[kRanks], uint64_t (&to)[kRanks]) {
   const uint32_t tid = threadIdx.x;
   uint64_t mineFrom = 0, mineTo = 0;
   for (uint32_t base = 0; base < a.cpSize; base += 8) {
@@ -57,7 +55,7 @@ __device__ __forceinline__ void move_statistics(const DirectExchangeArgs& a, uin
       }
     }
   }
-  if (tid < kMaxCpSize) {
+  if (tid < kRanks) {
     from[tid] = mineFrom;
     to[tid] = mineTo;
   }
@@ -67,7 +65,7 @@ __device__ __forceinline__ void move_statistics(const DirectExchangeArgs& a, uin
   uint64_t dst[kPerThread];
 #pragma unroll
   for (int i = 0; i < kPerThread; ++i) {
-    const uint32_t j = (blockIdx.x * kPerThread + i) * kBlockThreads + threadIdx.x;
+    const uint32_t j = (blockIdx.x * kPerThread + i) * kThreads + threadIdx.x;
     dst[i] = 0;
     if (j < a.pieces) {
       const uint32_t row = fast_div_by(j, a.byRowPieces);  // (e * cp + r) * cp + s
@@ -88,16 +86,15 @@ __device__ __forceinline__ void move_statistics(const DirectExchangeArgs& a, uin
 
 // A wavefront moves one access, 64 units = 1 KiB, of one (sender s, receiver r) pair: both tensors are
 // wave-uniform, and the launch is as many short wavefronts as there are KiB (two or four accesses per wavefront
-// measured 0-4 % slower from 64 MB up and the same below). Consecutive wavefronts take consecutive receivers, so a
-// workgroup reads neighbouring rows of one tensor and the launch sweeps all tensors in order; where a row is
-// shorter than an access, a workgroup takes four consecutive accesses of one pair instead (cp = 16 rows of 512 bytes
-// 46.3 -> 43.7 us; rows of 2 KiB stay with the receivers side by side: 512 tokens per rank more 44.9 -> 48.0 us).
-template <int kStatsPerThread, int kAuxLoad, int kAuxStore>
-__global__ __launch_bounds__(kBlockThreads) void helix_direct_exchange_kernel(DirectExchangeArgs a) {
-  __shared__ uint64_t from[kMaxCpSize], to[kMaxCpSize];
-  if (blockIdx.x < a.statsBlocks) return move_statistics<kStatsPerThread>(a, from, to);
+// measured 0-4 % slower from 64 MB up and the same below). Groups of 2^groupShift consecutive wavefronts take
+// consecutive accesses of one pair, consecutive groups consecutive receivers, so that the launch sweeps all tensors in
+// order.
+template <int kRanks, int kWaves, int kStatsPerThread, int kAuxLoad, int kAuxStore>
+__global__ __launch_bounds__(kWaves * kWaveLanes) void helix_direct_exchange_kernel(DirectExchangeArgs<kRanks> a) {
+  __shared__ uint64_t from[kRanks], to[kRanks];
+  if (blockIdx.x < a.statsBlocks) return move_statistics<kRanks, kWaves * kWaveLanes, kStatsPerThread>(a, from, to);
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWaveLanes);
-  const uint32_t w = (blockIdx.x - a.statsBlocks) * kBlockWaves + wave;
+  const uint32_t w = (blockIdx.x - a.statsBlocks) * kWaves + wave;
   if (w >= a.waves) return;
   const uint32_t pairs = w >> a.groupShift;
   const uint32_t t = fast_div_by(pairs, a.byCp);
@@ -123,6 +120,8 @@ __global__ __launch_bounds__(kBlockThreads) void helix_direct_exchange_kernel(Di
 // of the senders' tensors that belong to it, so an input row is read once and only the weighted sum is written.
 // Bound by the reads (cp input bytes for one written); no FIFO lines: cp = 8, T = 256, 8 heads of 128 per rank
 // 20.9 -> 6.6 us, T = 128, 16 heads of 512 71 -> 27 us (5.6 TB/s), cp = 16, T = 1024, 2 heads of 128 73 -> 27.6 us.
+
+constexpr int kCombineWaves = 4;  // wavefronts of a workgroup
 
 // Pieces of kWords * 2 elements.
 template <int kDtype, int kWords>
@@ -180,17 +179,17 @@ struct Piece<kDtype, 2> {
 // head. G = 4, 8, 16 or 32 lanes serve a slot for up to as many ranks. The payload loads are behind the statistics
 // loads and in front of the softmax, up to eight ranks' pieces in flight (sixteen at a time for sixteen ranks: the same).
 template <int kDtype, int kLanesPerSlot, int kWords, int kAuxLoad, int kAuxStore>
-__global__ __launch_bounds__(kBlockThreads) void helix_direct_combine_kernel(DirectCombineArgs a) {
+__global__ __launch_bounds__(kCombineWaves * kWaveLanes) void helix_direct_combine_kernel(DirectCombineArgs<kLanesPerSlot> a) {
   using P = Piece<kDtype, kWords>;
   constexpr uint32_t kPieceSize = kWords * 4;
   constexpr uint32_t kElements = kWords * 2;
   constexpr int kMaxSlots = kWords == 4 ? 17 : 9;  // heads that 64 pieces touch: a head is 32 elements or more
   constexpr uint32_t kSlotsPerPass = kWaveLanes / kLanesPerSlot;
   constexpr int kGroup = kLanesPerSlot < 8 ? kLanesPerSlot : 8;
-  __shared__ float __attribute__((aligned(16))) weights[kBlockWaves][kMaxSlots][kLanesPerSlot];
+  __shared__ float __attribute__((aligned(16))) weights[kCombineWaves][kMaxSlots][kLanesPerSlot];
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWaveLanes);
   const uint32_t lane = threadIdx.x % kWaveLanes;
-  const uint32_t w = blockIdx.x * kBlockWaves + wave;
+  const uint32_t w = blockIdx.x * kCombineWaves + wave;
   if (w >= a.waves) return;
   const uint32_t chunk = fast_div_by(w, a.byCp);
   const uint32_t r = w - chunk * a.cpSize;
@@ -303,11 +302,19 @@ constexpr uint64_t kStreamingBytes = 75ull << 20;
 // one thread (pointers, load, store), not for memory (cp = 4, T = 64: 3.4 -> 2.7 us; an empty kernel takes 2.1).
 constexpr uint32_t kShortStatsPieces = 65536;
 
+// A launch of rows of an access or more that reads more payload than this is made of workgroups of one wavefront, in
+// groups of four accesses of a pair: a slot is taken again as soon as one wavefront is done (134 MB in rows of 16 KiB
+// 45.8 -> 43.3 us, of 2 KiB 45.2 -> 42.5; a plain copy of as much from one piece of memory to another takes 42).
+// Below, a launch is bound by how fast its workgroups start and has four wavefronts in each (34 MB 11.0 -> 11.0 us, on
+// one set of tensors 9.0 -> 8.8, 8 MB 3.8 -> 3.5), consecutive receivers side by side. Rows shorter than an access have
+// four wavefronts, all of one pair, at any size: their statistics rows are short too, and the more of them a workgroup
+// holds the fewer lines are asked for twice (cp = 16, rows of 512 bytes, 134 MB: 43.6 us; with one wavefront 48.2).
+constexpr uint64_t kManyWorkgroupsBytes = 48ull << 20;
+
 // Wavefronts of a launch, at most: larger exchanges go out as several launches of consecutive entries.
 constexpr uint64_t kMaxLaunchWaves = 1ull << 25;
 
-static void set_ranks(DirectRanks& d, const KernelArgs& a, const uint64_t* broken) {
-  for (int r = 0; r < a.cpSize; ++r) d.rank[r] = a.rank[r];
+static void set_common(DirectCommon& d, const KernelArgs& a, const uint64_t* broken) {
   d.broken = broken;
   d.status = a.status;
   d.cpSize = static_cast<uint32_t>(a.cpSize);
@@ -319,18 +326,34 @@ static void set_ranks(DirectRanks& d, const KernelArgs& a, const uint64_t* broke
   d.recvBytes0 = a.recvBytes0;
   d.byCp = fast_div(d.cpSize);
 }
-static bool streams_payload(const KernelArgs& a) { return static_cast<uint64_t>(a.cpSize) * a.sendBytes0 > kStreamingBytes; }
+static uint64_t payload_bytes(const KernelArgs& a) { return static_cast<uint64_t>(a.cpSize) * a.sendBytes0; }
 
-hipError_t launch_direct_exchange(const KernelArgs& a, const uint64_t* broken, hipStream_t stream) {
-  DirectExchangeArgs d{};
-  set_ranks(d, a, broken);
+template <int kRanks, int kWaves, int kStatsPerThread, int kAuxLoad>
+static hipError_t launch_exchange_kernel(DirectExchangeArgs<kRanks>& d, uint32_t chunks, bool wholeLines, hipStream_t stream) {
+  constexpr uint32_t kPiecesPerBlock = kStatsPerThread * kWaves * kWaveLanes;
+  const uint32_t group = 1u << d.groupShift;
+  d.statsBlocks = (d.pieces + kPiecesPerBlock - 1) / kPiecesPerBlock;
+  d.waves = (chunks + group - 1) / group * group * d.cpSize * d.cpSize;
+  const dim3 blocks(d.statsBlocks + (d.waves + kWaves - 1) / kWaves), threads(kWaves * kWaveLanes);
+  if (wholeLines)
+    hipLaunchKernelGGL((helix_direct_exchange_kernel<kRanks, kWaves, kStatsPerThread, kAuxLoad, kAuxNtSc1>), blocks, threads, 0, stream, d);
+  else
+    hipLaunchKernelGGL((helix_direct_exchange_kernel<kRanks, kWaves, kStatsPerThread, kAuxLoad, kAuxNt>), blocks, threads, 0, stream, d);
+  return hipGetLastError();
+}
+
+template <int kRanks>
+static hipError_t launch_exchange_ranks(const KernelArgs& a, const uint64_t* broken, hipStream_t stream) {
+  DirectExchangeArgs<kRanks> d{};
+  set_common(d, a, broken);
   const uint32_t cp = d.cpSize;
   d.rowUnits = static_cast<uint32_t>(a.field0Bytes) / kUnitBytes;
   d.byRowUnits = fast_div(d.rowUnits);
   d.rowPieces = static_cast<uint32_t>(a.field1Bytes) / kPieceBytes;
   d.byRowPieces = fast_div(d.rowPieces);
-  d.groupShift = a.field0Bytes < kWaveLanes * kUnitBytes ? 2 : 0;
-  const bool streaming = streams_payload(a);
+  const bool shortRows = a.field0Bytes < kWaveLanes * kUnitBytes;
+  const bool streaming = payload_bytes(a) > kStreamingBytes, manyWorkgroups = payload_bytes(a) > kManyWorkgroupsBytes && !shortRows;
+  d.groupShift = manyWorkgroups || shortRows ? 2 : 0;
   // Rows of whole 128-byte lines are written through (their lines are complete with one store: rows of 2 KiB 11.0 ->
   // 10.1 us, of 512 bytes 46.0 -> 43.5); others leave it to the L2 to put the halves of a line together (rows of 480
   // bytes 9.8 us written through, 9.2 left there).
@@ -353,53 +376,32 @@ hipError_t launch_direct_exchange(const KernelArgs& a, const uint64_t* broken, h
     d.recvBytes0 = entries * cp * d.recvStride0;
     d.units = entries * d.rowUnits;
     d.pieces = entries * cp * cp * d.rowPieces;
-    const bool shortStats = !streaming && d.pieces <= kShortStatsPieces;
-    const uint32_t piecesPerBlock = (shortStats ? 1 : 4) * kBlockThreads;
-    d.statsBlocks = (d.pieces + piecesPerBlock - 1) / piecesPerBlock;
-    const uint32_t group = 1u << d.groupShift;
     const uint32_t chunks = (d.units + kWaveLanes - 1) / kWaveLanes;
-    d.waves = (chunks + group - 1) / group * group * cp * cp;
-    const dim3 blocks(d.statsBlocks + (d.waves + kBlockWaves - 1) / kBlockWaves);
-#define HELIX_LAUNCH_DIRECT(P, L, S) hipLaunchKernelGGL((helix_direct_exchange_kernel<P, L, S>), blocks, dim3(kBlockThreads), 0, stream, d)
-    if (streaming && wholeLines) HELIX_LAUNCH_DIRECT(4, kAuxNt, kAuxNtSc1);
-    else if (streaming) HELIX_LAUNCH_DIRECT(4, kAuxNt, kAuxNt);
-    else if (shortStats && wholeLines) HELIX_LAUNCH_DIRECT(1, kAuxNone, kAuxNtSc1);
-    else if (shortStats) HELIX_LAUNCH_DIRECT(1, kAuxNone, kAuxNt);
-    else if (wholeLines) HELIX_LAUNCH_DIRECT(4, kAuxNone, kAuxNtSc1);
-    else HELIX_LAUNCH_DIRECT(4, kAuxNone, kAuxNt);
-#undef HELIX_LAUNCH_DIRECT
-    const hipError_t err = hipGetLastError();
+    hipError_t err;
+    if (manyWorkgroups && streaming) err = launch_exchange_kernel<kRanks, 1, 4, kAuxNt>(d, chunks, wholeLines, stream);
+    else if (manyWorkgroups) err = launch_exchange_kernel<kRanks, 1, 4, kAuxNone>(d, chunks, wholeLines, stream);
+    else if (streaming) err = launch_exchange_kernel<kRanks, 4, 4, kAuxNt>(d, chunks, wholeLines, stream);
+    else if (d.pieces <= kShortStatsPieces) err = launch_exchange_kernel<kRanks, 4, 1, kAuxNone>(d, chunks, wholeLines, stream);
+    else err = launch_exchange_kernel<kRanks, 4, 4, kAuxNone>(d, chunks, wholeLines, stream);
     if (err != hipSuccess) return err;
   }
   return hipSuccess;
 }
 
-template <int kDtype, int kWords, int kAuxLoad, int kAuxStore>
-static void launch_combine_kernel(const DirectCombineArgs& d, hipStream_t stream) {
-  const dim3 blocks((d.waves + kBlockWaves - 1) / kBlockWaves), threads(kBlockThreads);
-#define HELIX_LAUNCH_COMBINE(G) hipLaunchKernelGGL((helix_direct_combine_kernel<kDtype, G, kWords, kAuxLoad, kAuxStore>), blocks, threads, 0, stream, d)
-  if (d.cpSize <= 4) HELIX_LAUNCH_COMBINE(4);
-  else if (d.cpSize <= 8) HELIX_LAUNCH_COMBINE(8);
-  else if (d.cpSize <= 16) HELIX_LAUNCH_COMBINE(16);
-  else HELIX_LAUNCH_COMBINE(32);
-#undef HELIX_LAUNCH_COMBINE
+hipError_t launch_direct_exchange(const KernelArgs& a, const uint64_t* broken, hipStream_t stream) {
+  return a.cpSize <= 8    ? launch_exchange_ranks<8>(a, broken, stream)
+         : a.cpSize <= 16 ? launch_exchange_ranks<16>(a, broken, stream)
+                          : launch_exchange_ranks<32>(a, broken, stream);
 }
 
-template <int kDtype, int kWords>
-static void launch_combine_kernel(const DirectCombineArgs& d, bool streaming, hipStream_t stream) {
-  // a result that fits beside its inputs is written through (T = 256: 6.8 -> 6.5 us); one behind a stream of inputs is not
-  // (T = 128, 16 heads of 512: 27.1, written through 27.6)
-  if (streaming) launch_combine_kernel<kDtype, kWords, kAuxNt, kAuxNt>(d, stream);
-  else launch_combine_kernel<kDtype, kWords, kAuxNone, kAuxNtSc1>(d, stream);
-}
-
-hipError_t launch_direct_combine(const KernelArgs& a, const uint64_t* broken, hipStream_t stream) {
-  DirectCombineArgs d{};
-  set_ranks(d, a, broken);
-  const bool wide = a.headDim % 8 == 0;
-  const uint32_t pieceSize = wide ? 16 : 8;
-  d.rowPieces = static_cast<uint32_t>(a.field0Bytes) / pieceSize;
-  d.headPieces = static_cast<uint32_t>(a.headDim) * 2u / pieceSize;
+template <int kLanesPerSlot, int kDtype, int kWords>
+static hipError_t launch_combine_kernel(const KernelArgs& a, const uint64_t* broken, hipStream_t stream) {
+  DirectCombineArgs<kLanesPerSlot> d{};
+  set_common(d, a, broken);
+  for (uint32_t r = 0; r < d.cpSize; ++r) d.rank[r] = a.rank[r];
+  constexpr uint32_t kPieceSize = kWords * 4;
+  d.rowPieces = static_cast<uint32_t>(a.field0Bytes) / kPieceSize;
+  d.headPieces = static_cast<uint32_t>(a.headDim) * 2u / kPieceSize;
   d.heads = static_cast<uint32_t>(a.heads);
   d.byHeadPieces = fast_div(d.headPieces);
   d.byHeads = fast_div(d.heads);
@@ -407,12 +409,29 @@ hipError_t launch_direct_combine(const KernelArgs& a, const uint64_t* broken, hi
   d.statsMode = a.statsMode;
   d.lseBase2 = a.lseBase2;
   d.waves = (d.outPieces + kWaveLanes - 1) / kWaveLanes * d.cpSize;  // at most 2^22: a rank's output is < 2 GiB / cp
-  const bool streaming = streams_payload(a);
-  if (a.dtype == 0)
-    wide ? launch_combine_kernel<0, 4>(d, streaming, stream) : launch_combine_kernel<0, 2>(d, streaming, stream);
+  const dim3 blocks((d.waves + kCombineWaves - 1) / kCombineWaves), threads(kCombineWaves * kWaveLanes);
+  // a result that fits beside its inputs is written through (T = 256: 6.8 -> 6.5 us); one behind a stream of inputs is not
+  // (T = 128, 16 heads of 512: 27.1, written through 27.6)
+  if (payload_bytes(a) > kStreamingBytes)
+    hipLaunchKernelGGL((helix_direct_combine_kernel<kDtype, kLanesPerSlot, kWords, kAuxNt, kAuxNt>), blocks, threads, 0, stream, d);
   else
-    wide ? launch_combine_kernel<1, 4>(d, streaming, stream) : launch_combine_kernel<1, 2>(d, streaming, stream);
+    hipLaunchKernelGGL((helix_direct_combine_kernel<kDtype, kLanesPerSlot, kWords, kAuxNone, kAuxNtSc1>), blocks, threads, 0, stream, d);
   return hipGetLastError();
+}
+
+template <int kLanesPerSlot>
+static hipError_t launch_combine_ranks(const KernelArgs& a, const uint64_t* broken, hipStream_t stream) {
+  const bool wide = a.headDim % 8 == 0;
+  if (a.dtype == 0)
+    return wide ? launch_combine_kernel<kLanesPerSlot, 0, 4>(a, broken, stream) : launch_combine_kernel<kLanesPerSlot, 0, 2>(a, broken, stream);
+  return wide ? launch_combine_kernel<kLanesPerSlot, 1, 4>(a, broken, stream) : launch_combine_kernel<kLanesPerSlot, 1, 2>(a, broken, stream);
+}
+
+hipError_t launch_direct_combine(const KernelArgs& a, const uint64_t* broken, hipStream_t stream) {
+  return a.cpSize <= 4    ? launch_combine_ranks<4>(a, broken, stream)
+         : a.cpSize <= 8  ? launch_combine_ranks<8>(a, broken, stream)
+         : a.cpSize <= 16 ? launch_combine_ranks<16>(a, broken, stream)
+                          : launch_combine_ranks<32>(a, broken, stream);
 }
 
 }  // namespace helix

@@ -59,8 +59,12 @@ CASES = [
     (8, 64, 1024, 16, 64),      # whole lines
     (8, 64, 1024, 16, 4),       # ... but outputs that start inside a line
     (32, 9, 128, 8, 0),
-    (8, 300, 2048, 16, 0),      # 160 MB in and out: payload past the memory-side cache
-    (8, 300, 2056, 16, 0),      # ... with rows that are no whole lines
+    (8, 385, 1024, 16, 0),      # 50 MB: workgroups of one wavefront
+    (9, 311, 1032, 2, 0),       # ... ragged, rows that are no whole lines
+    (8, 3100, 128, 2, 0),       # ... but not for rows shorter than an access
+    (8, 301, 2048, 16, 0),      # 79 MB: payload past the memory-side cache
+    (16, 680, 256, 4, 0),       # ... in short rows
+    (8, 301, 2056, 16, 0),      # ... with rows that are no whole lines
     (8, 80, 8192, 2, 0),        # ... and few statistics
     (32, 33000, 8, 2, 0),       # more entries than one launch takes
 ]
