@@ -249,6 +249,15 @@ void launch(const char* what, F&& call) {
   if (rc != 0) raise_last(what);
 }
 
+// c10::DeviceGuard asks for the device on its way in and out; where the device is current already, once is enough.
+struct OnDevice {
+  c10::OptionalDeviceGuard guard;
+  explicit OnDevice(const at::Device& device) {
+    int current = -1;
+    if (hipGetDevice(&current) != hipSuccess || current != device.index()) guard.reset_device(device);
+  }
+};
+
 hipStream_t current_stream(const at::Device& device) { return c10::hip::getCurrentHIPStream(device.index()).stream(); }
 
 // ---------------------------------------------------------------------------
@@ -268,7 +277,7 @@ PyObject* alltoall_loopback(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     const at::Tensor &o0 = os.at(0), &s0 = ss.at(0);
     const Shape shape = check_pair(o0, s0, cp);
     const at::Device device = ws.device();
-    const c10::DeviceGuard guard(device);
+    const OnDevice on(device);
 
     Outputs outO, outS;
     PyObject *givenO = nullptr, *givenS = nullptr;
@@ -357,7 +366,7 @@ PyObject* alltoall_combine_loopback(PyObject*, PyObject* const* args, Py_ssize_t
     require(shape.row0 % heads == 0 && (shape.row0 / heads) % 4 == 0 && shape.row0 / heads >= 32,
             "partial_o rows must hold heads * head_dim elements, head_dim a multiple of 4 and >= 32");
     const at::Device device = ws.device();
-    const c10::DeviceGuard guard(device);
+    const OnDevice on(device);
 
     Outputs combined, lse;
     if (o0.dim() == 4 && o0.size(1) == cp && o0.size(2) == heads)
@@ -413,7 +422,7 @@ PyObject* dcp_reduce(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int returnLse = PyObject_IsTrue(args[3]), base2 = PyObject_IsTrue(args[5]);
     if (returnLse < 0 || base2 < 0) throw PythonError{};
     const int channels = as_int(args[4]);
-    const c10::DeviceGuard guard(device);
+    const OnDevice on(device);
 
     Outputs combined(n, {b, hp, d}, o0.scalar_type(), device), lse;
     if (returnLse) lse = Outputs(n, {b, hp}, at::kFloat, device);
@@ -628,10 +637,34 @@ Group* group_of(const at::Tensor& ws, int cp) {
   return reinterpret_cast<Group*>(found);
 }
 
-// alltoall(partial_o, softmax_stats, workspace, cp_rank, cp_size)
-PyObject* alltoall(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+// The five arguments of alltoall, by position or name.
+constexpr int kAlltoallArgs = 5;
+const char* const kAlltoallNames[kAlltoallArgs] = {"partial_o", "softmax_stats", "workspace", "cp_rank", "cp_size"};
+
+void parse_alltoall(PyObject* const* args, Py_ssize_t nargs, PyObject* names, PyObject* (&out)[kAlltoallArgs]) {
+  const Py_ssize_t keywords = names ? PyTuple_GET_SIZE(names) : 0;
+  auto type_error = [](const std::string& message) {
+    PyErr_SetString(PyExc_TypeError, ("alltoall() " + message).c_str());
+    throw PythonError{};
+  };
+  if (nargs > kAlltoallArgs) type_error("takes 5 arguments (" + std::to_string(nargs) + " given)");
+  for (int i = 0; i < kAlltoallArgs; ++i) out[i] = i < nargs ? args[i] : nullptr;
+  for (Py_ssize_t k = 0; k < keywords; ++k) {
+    PyObject* name = PyTuple_GET_ITEM(names, k);
+    int i = 0;
+    while (i < kAlltoallArgs && PyUnicode_CompareWithASCIIString(name, kAlltoallNames[i]) != 0) ++i;
+    if (i == kAlltoallArgs) type_error("got an unexpected keyword argument");
+    if (out[i]) type_error(std::string("got multiple values for argument '") + kAlltoallNames[i] + "'");
+    out[i] = args[nargs + k];
+  }
+  for (int i = 0; i < kAlltoallArgs; ++i)
+    if (!out[i]) type_error(std::string("missing required argument '") + kAlltoallNames[i] + "'");
+}
+
+PyObject* alltoall(PyObject*, PyObject* const* positional, Py_ssize_t nargs, PyObject* names) {
   return guarded([&]() -> PyObject* {
-    require(nargs == 5, "alltoall takes 5 arguments");
+    PyObject* args[kAlltoallArgs];
+    parse_alltoall(positional, nargs, names, args);
     const int rank = as_int(args[3]), cp = as_int(args[4]);
     require(cp >= 1 && cp <= kMaxCp, "cp_size must be in [1, 32]");
     const at::Tensor& o = as_tensor(args[0], "partial_o and softmax_stats must be tensors");
@@ -642,7 +675,6 @@ PyObject* alltoall(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     require(rank >= 0 && rank < cp, "cp_rank must be in [0, cp_size)");
     const at::Device device = ws.device();
     require(device == o.device() && device == s.device(), "all tensors must live on one device");
-    const c10::DeviceGuard guard(device);
 
     Group* group = group_of(ws, cp);
     Exchange* ex = group->ex;
@@ -661,6 +693,7 @@ PyObject* alltoall(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
       while (!(ex->called & (1u << peer))) ++peer;
       require(same_pair(o, s, ex->o[peer], ex->s[peer]), "logical ranks of one group must exchange tensors of one shape and dtype");
     } else {
+      const OnDevice on(device);
       std::unique_ptr<Exchange> fresh(new Exchange);
       fresh->channels = env_channel_count();
       fresh->maxChannels = device_max_channels(cp);
@@ -689,6 +722,7 @@ PyObject* alltoall(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
                 ex->workspace, ex->channels, ex->maxChannels);
     const hipStream_t stream = current_stream(device);
     if (ex->eager) {
+      const OnDevice on(device);
       int rc;
       {
         std::lock_guard<std::mutex> lock(g_launchMutex);
@@ -718,6 +752,7 @@ PyObject* alltoall(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
     group->ex = nullptr;  // the next exchange may start while this one is being enqueued
     try {
+      const OnDevice on(device);
       flush(*ex, cp, stream);
     } catch (...) {
       Py_DECREF(result);
@@ -759,11 +794,28 @@ PyObject* bind(PyObject*, PyObject* args) {
   Py_RETURN_NONE;
 }
 
-PyCFunction fast(_PyCFunctionFast f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)); }
+PyDoc_STRVAR(alltoall_doc,
+             "alltoall(partial_o, softmax_stats, workspace, cp_rank, cp_size)\n"
+             "--\n"
+             "\n"
+             "Helix all-to-all of one rank.\n"
+             "\n"
+             "``partial_o`` is ``[..., cp_size, D]`` (fp16/bf16), ``softmax_stats`` is\n"
+             "``[..., cp_size, S]`` (fp32, S even); slice ``[..., p, :]`` goes to rank\n"
+             "``p``. Returns tensors of the same shapes whose slice ``[..., p, :]`` came\n"
+             "from rank ``p``: ``out_r[e, s, :] = in_s[e, r, :]``, bit for bit.\n"
+             "Asynchronous on the current stream. With the ranks of one device the\n"
+             "returned tensors are filled once every rank has called (see the module\n"
+             "docstring for what that asks of the inputs).");
+
+template <class F>
+PyCFunction fast(F f) {
+  return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f));
+}
 
 PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, nullptr},
-    {"alltoall", fast(alltoall), METH_FASTCALL, nullptr},
+    {"alltoall", fast(alltoall), METH_FASTCALL | METH_KEYWORDS, alltoall_doc},
     {"alltoall_loopback", fast(alltoall_loopback), METH_FASTCALL, nullptr},
     {"alltoall_combine_loopback", fast(alltoall_combine_loopback), METH_FASTCALL, nullptr},
     {"dcp_reduce", fast(dcp_reduce), METH_FASTCALL, nullptr},

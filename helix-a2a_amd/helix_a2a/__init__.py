@@ -27,7 +27,7 @@ import torch
 
 from helix_a2a import _ops
 from helix_a2a._ops import STATS_LSE, STATS_LSE_PACKED, STATS_MAX_SUM  # noqa: F401
-from helix_a2a._native import alltoall as _alltoall
+from helix_a2a._native import alltoall  # noqa: F401  -- called once per rank: no Python frame in between
 from helix_a2a._native import alltoall_combine_loopback as _alltoall_combine_loopback
 from helix_a2a._native import alltoall_loopback as _alltoall_loopback
 from helix_a2a._native import dcp_reduce as _dcp_reduce
@@ -89,26 +89,6 @@ def init_workspace(workspace: torch.Tensor, cp_rank: int, cp_size: int) -> None:
     """
     _ops.initialize_workspace(workspace, cp_rank, cp_size)
     torch.cuda.current_stream().synchronize()
-
-
-def alltoall(
-    partial_o: torch.Tensor,
-    softmax_stats: torch.Tensor,
-    workspace: torch.Tensor,
-    cp_rank: int,
-    cp_size: int,
-) -> Tuple[torch.Tensor, torch.Tensor]:
-    """Helix all-to-all of one rank.
-
-    ``partial_o`` is ``[..., cp_size, D]`` (fp16/bf16), ``softmax_stats`` is
-    ``[..., cp_size, S]`` (fp32, S even); slice ``[..., p, :]`` goes to rank
-    ``p``. Returns tensors of the same shapes whose slice ``[..., p, :]`` came
-    from rank ``p``: ``out_r[e, s, :] = in_s[e, r, :]``, bit for bit.
-    Asynchronous on the current stream. With the ranks of one device the
-    returned tensors are filled once every rank has called (see the module
-    docstring for what that asks of the inputs).
-    """
-    return _alltoall(partial_o, softmax_stats, workspace, cp_rank, cp_size)
 
 
 def alltoall_loopback(
