@@ -11,6 +11,7 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/hip/impl/HIPCachingAllocatorMasqueradingAsCUDA.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -185,29 +186,26 @@ int device_max_channels(int cp) {
   return n;
 }
 
-// One allocation for the outputs of all ranks, rank r's is slice r.
+// One allocation for the outputs of all ranks, rank r's is slice r. It comes straight from torch's caching allocator, on
+// the current device and stream (an at::empty and a view of it per rank cost 1 us of a call more).
 struct Outputs {
-  at::Tensor all;
+  c10::Storage storage;
+  caffe2::TypeMeta dtype;
   std::vector<int64_t> sizes;  // of a slice
   int64_t numel = 1;
   Outputs() = default;
-  Outputs(int cp, at::IntArrayRef slice, at::ScalarType dtype, const at::Device& device) : sizes(slice.vec()) {
-    std::vector<int64_t> full;
-    full.reserve(slice.size() + 1);
-    full.push_back(cp);
-    for (int64_t d : slice) {
-      full.push_back(d);
-      numel *= d;
-    }
-    all = at::empty(full, at::TensorOptions().dtype(dtype).device(device));
+  Outputs(int cp, at::IntArrayRef slice, at::ScalarType type) : dtype(c10::scalarTypeToTypeMeta(type)), sizes(slice.vec()) {
+    for (int64_t d : slice) numel *= d;
+    storage = c10::Storage(c10::make_intrusive<c10::StorageImpl>(c10::StorageImpl::use_byte_size_t(), static_cast<size_t>(cp * numel) * dtype.itemsize(),
+                                                                 c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get(), /*resizable=*/true));
   }
   at::Tensor slice(int r) const {
-    at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::TensorImpl::VIEW, c10::Storage(all.storage()), all.key_set(), all.dtype());
+    at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(storage), c10::DispatchKeySet(c10::DispatchKey::CUDA), dtype);
     t.unsafeGetTensorImpl()->set_storage_offset(r * numel);
     t.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
     return t;
   }
-  void* data(int r) const { return static_cast<char*>(all.data_ptr()) + r * numel * static_cast<int64_t>(all.element_size()); }
+  void* data(int r) const { return static_cast<char*>(storage.mutable_data()) + r * numel * static_cast<int64_t>(dtype.itemsize()); }
 };
 
 PyObject* wrap_slices(const Outputs& out, int cp) {
@@ -282,8 +280,8 @@ PyObject* alltoall_loopback(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     Outputs outO, outS;
     PyObject *givenO = nullptr, *givenS = nullptr;
     if (args[4] == Py_None) {
-      outO = Outputs(cp, o0.sizes(), o0.scalar_type(), device);
-      outS = Outputs(cp, s0.sizes(), at::kFloat, device);
+      outO = Outputs(cp, o0.sizes(), o0.scalar_type());
+      outS = Outputs(cp, s0.sizes(), at::kFloat);
     } else {
       PyObject* seq = PySequence_Fast(args[4], "out must be a pair of sequences");
       if (!seq) throw PythonError{};
@@ -370,10 +368,10 @@ PyObject* alltoall_combine_loopback(PyObject*, PyObject* const* args, Py_ssize_t
 
     Outputs combined, lse;
     if (o0.dim() == 4 && o0.size(1) == cp && o0.size(2) == heads)
-      combined = Outputs(cp, {shape.entries, heads, shape.row0 / heads}, o0.scalar_type(), device);
+      combined = Outputs(cp, {shape.entries, heads, shape.row0 / heads}, o0.scalar_type());
     else
-      combined = Outputs(cp, {shape.entries, shape.row0}, o0.scalar_type(), device);
-    if (returnLse) lse = Outputs(cp, {shape.entries, heads}, at::kFloat, device);
+      combined = Outputs(cp, {shape.entries, shape.row0}, o0.scalar_type());
+    if (returnLse) lse = Outputs(cp, {shape.entries, heads}, at::kFloat);
     helix_a2a_params_t params[kMaxCp];
     helix_a2a_combine_out_t out[kMaxCp];
     const int maxChannels = device_max_channels(cp);
@@ -424,8 +422,8 @@ PyObject* dcp_reduce(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     const int channels = as_int(args[4]);
     const OnDevice on(device);
 
-    Outputs combined(n, {b, hp, d}, o0.scalar_type(), device), lse;
-    if (returnLse) lse = Outputs(n, {b, hp}, at::kFloat, device);
+    Outputs combined(n, {b, hp, d}, o0.scalar_type()), lse;
+    if (returnLse) lse = Outputs(n, {b, hp}, at::kFloat);
     std::vector<at::Tensor> keep;  // contiguous copies, until the launch is enqueued
     helix_a2a_params_t params[kMaxCp];
     helix_a2a_combine_out_t out[kMaxCp];
@@ -703,8 +701,8 @@ PyObject* alltoall(PyObject*, PyObject* const* positional, Py_ssize_t nargs, PyO
       fresh->eager = g_eagerSend;
       fresh->started = now_seconds();
       fresh->workspace = ws;
-      fresh->outO = Outputs(cp, o.sizes(), o.scalar_type(), device);
-      fresh->outS = Outputs(cp, s.sizes(), at::kFloat, device);
+      fresh->outO = Outputs(cp, o.sizes(), o.scalar_type());
+      fresh->outS = Outputs(cp, s.sizes(), at::kFloat);
       ex = fresh.release();
     }
     // from here on `ex` belongs to the group, or goes with this call
