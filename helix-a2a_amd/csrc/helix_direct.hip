@@ -119,9 +119,10 @@ __global__ __launch_bounds__(kWaves * kWaveLanes) void helix_direct_exchange_ker
 // The exchange and the combine after it in one pass: a lane makes one piece of one rank's output from the cp pieces
 // of the senders' tensors that belong to it, so an input row is read once and only the weighted sum is written.
 // Bound by the reads (cp input bytes for one written); no FIFO lines: cp = 8, T = 256, 8 heads of 128 per rank
-// 20.9 -> 6.6 us, T = 128, 16 heads of 512 71 -> 27 us (5.6 TB/s), cp = 16, T = 1024, 2 heads of 128 73 -> 27.6 us.
+// 20.9 -> 5.5 us, T = 128, 16 heads of 512 71 -> 25.5 us (6.0 TB/s), cp = 16, T = 1024, 2 heads of 128 73 -> 25.7 us.
 
 constexpr int kCombineWaves = 4;  // wavefronts of a workgroup
+constexpr int kXcdRun = 64;       // consecutive workgroups' worth of pieces one XCD takes, at most
 
 // Pieces of kWords * 2 elements.
 template <int kDtype, int kWords>
@@ -169,6 +170,23 @@ struct Piece<kDtype, 2> {
   }
 };
 
+// The reduction of a value over aligned groups of 4, 8, 16 or 32 lanes, in every lane of the group: neighbours trade
+// places within quads, then halves and rows of lanes are mirrored into each other (their lanes hold equal values by
+// then), without a trip through LDS. Thirty-two lanes take one.
+template <int kControl>
+__device__ __forceinline__ float dpp(float v) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), kControl, 0xF, 0xF, true));
+}
+template <int kLanes, class Op>
+__device__ __forceinline__ float reduce_lanes(float v, Op op) {
+  v = op(v, dpp<0xB1>(v));                        // quad_perm 1 0 3 2
+  v = op(v, dpp<0x4E>(v));                        // quad_perm 2 3 0 1
+  if (kLanes >= 8) v = op(v, dpp<0x141>(v));      // row_half_mirror
+  if (kLanes >= 16) v = op(v, dpp<0x140>(v));     // row_mirror
+  if (kLanes >= 32) v = op(v, shuffle_xor(v, 16));
+  return v;
+}
+
 // A wavefront makes 64 consecutive pieces of one rank's output (one per lane: two per lane measured the same at
 // large sizes and up to 25 % slower below, where wavefronts are few); consecutive wavefronts take consecutive ranks,
 // whose rows are neighbours in every input tensor.
@@ -177,7 +195,14 @@ struct Piece<kDtype, 2> {
 // (i / G)-th head the pieces touch ("slot") and sender i % G, loads that sender's log-sum-exp of that head, and a
 // softmax over the G lanes of the slot gives the weights, which go through LDS to the lanes that own pieces of the
 // head. G = 4, 8, 16 or 32 lanes serve a slot for up to as many ranks. The payload loads are behind the statistics
-// loads and in front of the softmax, up to eight ranks' pieces in flight (sixteen at a time for sixteen ranks: the same).
+// loads and in front of the softmax, four ranks' pieces at a time (eight: T = 256 5.5 -> 5.6 us, T = 512 13.2 -> 13.5,
+// the same above).
+//
+// Workgroups go to the XCDs in turn, and a wavefront reads the same place of every rank's tensor, tensors whose bases
+// agree in their lower bits as a rule. With consecutive workgroups on consecutive XCDs each XCD then sees a fixed part of
+// every 16 KiB of all of them, that is a part of the memory channels. Runs of 64 workgroups on one XCD (fewer in
+// launches of fewer than 512) cover all of it: cp = 16, T = 1024 28.2 -> 25.7 us, T = 2048, 4 heads of 128 28.1 -> 25.7, T = 128,
+// 16 heads of 512 26.5 -> 25.5, T = 512, 8 heads 14.2 -> 13.2, T = 256 on one set of tensors 6.2 -> 5.5.
 template <int kDtype, int kLanesPerSlot, int kWords, int kAuxLoad, int kAuxStore>
 __global__ __launch_bounds__(kCombineWaves * kWaveLanes) void helix_direct_combine_kernel(DirectCombineArgs<kLanesPerSlot> a) {
   using P = Piece<kDtype, kWords>;
@@ -185,11 +210,12 @@ __global__ __launch_bounds__(kCombineWaves * kWaveLanes) void helix_direct_combi
   constexpr uint32_t kElements = kWords * 2;
   constexpr int kMaxSlots = kWords == 4 ? 17 : 9;  // heads that 64 pieces touch: a head is 32 elements or more
   constexpr uint32_t kSlotsPerPass = kWaveLanes / kLanesPerSlot;
-  constexpr int kGroup = kLanesPerSlot < 8 ? kLanesPerSlot : 8;
+  constexpr int kGroup = 4;
   __shared__ float __attribute__((aligned(16))) weights[kCombineWaves][kMaxSlots][kLanesPerSlot];
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWaveLanes);
   const uint32_t lane = threadIdx.x % kWaveLanes;
-  const uint32_t w = blockIdx.x * kCombineWaves + wave;
+  const uint32_t block = blockIdx.x < a.groupedBlocks ? static_cast<uint32_t>(xcd_grouped(static_cast<int>(blockIdx.x), a.xcdGroup)) : blockIdx.x;
+  const uint32_t w = block * kCombineWaves + wave;
   if (w >= a.waves) return;
   const uint32_t chunk = fast_div_by(w, a.byCp);
   const uint32_t r = w - chunk * a.cpSize;
@@ -252,14 +278,11 @@ __global__ __launch_bounds__(kCombineWaves * kWaveLanes) void helix_direct_combi
     const bool serving = slot < slots && realSender;
     const float lse = serving ? lse_of_stats(sv.x, sv.y, a.statsMode == 2 ? 0 : a.statsMode, 0, a.lseBase2 != 0) : -INFINITY;
     float m = lse;
-#pragma unroll
-    for (int x = 1; x < kLanesPerSlot; x <<= 1) m = fmaxf(m, shuffle_xor(m, x));
+    m = reduce_lanes<kLanesPerSlot>(m, [](float x, float y) { return fmaxf(x, y); });
     if (m == -INFINITY) m = 0.0f;  // every rank masked: weights 0, log-sum-exp -inf
     float ex = fast_exp(lse - m);
     if (isnan(ex)) ex = 0.0f;
-    float total = ex;
-#pragma unroll
-    for (int x = 1; x < kLanesPerSlot; x <<= 1) total += shuffle_xor(total, x);
+    const float total = reduce_lanes<kLanesPerSlot>(ex, [](float x, float y) { return x + y; });
     // (ranks beyond cp get weight 0: their pieces are zeros, and 0 * 0 stays 0)
     if (slot < slots) weights[wave][slot][q] = ex * __builtin_amdgcn_rcpf(fmaxf(total, 1e-10f));
     float* lseOut = reinterpret_cast<float*>(a.rank[r].recv1);
@@ -410,6 +433,9 @@ static hipError_t launch_combine_kernel(const KernelArgs& a, const uint64_t* bro
   d.lseBase2 = a.lseBase2;
   d.waves = (d.outPieces + kWaveLanes - 1) / kWaveLanes * d.cpSize;  // at most 2^22: a rank's output is < 2 GiB / cp
   const dim3 blocks((d.waves + kCombineWaves - 1) / kCombineWaves), threads(kCombineWaves * kWaveLanes);
+  d.xcdGroup = kXcdRun;
+  while (d.xcdGroup > 1 && 8u * d.xcdGroup > blocks.x) d.xcdGroup /= 2;
+  d.groupedBlocks = blocks.x / (8 * d.xcdGroup) * (8 * d.xcdGroup);
   // a result that fits beside its inputs is written through (T = 256: 6.8 -> 6.5 us); one behind a stream of inputs is not
   // (T = 128, 16 heads of 512: 27.1, written through 27.6)
   if (payload_bytes(a) > kStreamingBytes)

@@ -55,6 +55,8 @@ struct DirectCombine {
   uint32_t headPieces;  // of a head
   uint32_t heads;       // heads of a row
   FastDiv byHeadPieces, byHeads;
+  int xcdGroup;            // consecutive workgroups' worth of pieces that one XCD takes (xcd_grouped) ...
+  uint32_t groupedBlocks;  // ... in the first so many workgroups, whole tiles of it
   int statsMode, lseBase2;
 };
 

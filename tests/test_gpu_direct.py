@@ -110,6 +110,10 @@ COMBINE_CASES = [
     (17, 9, 2, 64, torch.bfloat16, 1, False),    # thirty-two lanes to a head: several passes over the heads of an access
     (32, 6, 3, 32, torch.float16, 2, False),
     (8, 1, 1, 576, torch.bfloat16, 2, True),     # a head longer than an access
+    (8, 16, 1, 128, torch.float16, 1, False),    # eight workgroups: one to an XCD
+    (8, 18, 1, 128, torch.bfloat16, 1, False),   # ... and some more
+    (8, 1024, 1, 128, torch.bfloat16, 0, False), # 512 workgroups: runs of sixty-four to an XCD
+    (8, 1031, 1, 128, torch.float16, 1, False),  # ... and a rest as dispatched
     (8, 600, 8, 128, torch.bfloat16, 1, False),  # 79 MB of partial outputs: read past the memory-side cache
     (4, 640, 30, 132, torch.bfloat16, 1, False), # ... in 8-byte pieces
 ]
