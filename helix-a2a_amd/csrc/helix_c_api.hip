@@ -278,9 +278,9 @@ int build_plan(const helix_a2a_params_t* ranks, int count, bool exchangeOutputs,
                 f0 + f1, sh.lines, kFifoEntryLines);
 
   // everything above is pure argument checking; from here on the device is consulted
-  int cuCount = 0;
-  rc = resolve_cu_count(0, &cuCount);
-  if (rc) return rc;
+  DeviceState* st = nullptr;
+  if ((rc = device_state(&st))) return rc;
+  const int cuCount = st->cuCount;
   const int maxCh = builtin ? builtin->maxChannels : max_channel_count(cp, cuCount);
   if (builtin == nullptr) {
     if (p0.max_channel_count != maxCh)
@@ -307,9 +307,6 @@ int build_plan(const helix_a2a_params_t* ranks, int count, bool exchangeOutputs,
     channels = auto_channels(cp, p0.entry_count, cuCount);
     if (channels > maxCh) channels = maxCh;
   }
-
-  DeviceState* st = nullptr;
-  if ((rc = device_state(&st))) return rc;
 
   a.workspace = builtin ? builtin->base : reinterpret_cast<uint8_t*>(p0.workspace);
   a.rowStrideBytes = builtin ? builtin->rowStrideBytes : p0.workspace_stride_u64 * 8ull;

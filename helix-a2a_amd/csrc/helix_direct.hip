@@ -349,6 +349,11 @@ static void set_common(DirectCommon& d, const KernelArgs& a, const uint64_t* bro
   d.recvBytes0 = a.recvBytes0;
   d.byCp = fast_div(d.cpSize);
 }
+template <class Args>
+static hipError_t launch(void (*kernel)(Args), dim3 blocks, dim3 threads, Args& args, hipStream_t stream) {
+  void* params[] = {&args};
+  return hipLaunchKernel(reinterpret_cast<const void*>(kernel), blocks, threads, params, 0, stream);
+}
 static uint64_t payload_bytes(const KernelArgs& a) { return static_cast<uint64_t>(a.cpSize) * a.sendBytes0; }
 
 template <int kRanks, int kWaves, int kStatsPerThread, int kAuxLoad>
@@ -358,11 +363,8 @@ static hipError_t launch_exchange_kernel(DirectExchangeArgs<kRanks>& d, uint32_t
   d.statsBlocks = (d.pieces + kPiecesPerBlock - 1) / kPiecesPerBlock;
   d.waves = (chunks + group - 1) / group * group * d.cpSize * d.cpSize;
   const dim3 blocks(d.statsBlocks + (d.waves + kWaves - 1) / kWaves), threads(kWaves * kWaveLanes);
-  if (wholeLines)
-    hipLaunchKernelGGL((helix_direct_exchange_kernel<kRanks, kWaves, kStatsPerThread, kAuxLoad, kAuxNtSc1>), blocks, threads, 0, stream, d);
-  else
-    hipLaunchKernelGGL((helix_direct_exchange_kernel<kRanks, kWaves, kStatsPerThread, kAuxLoad, kAuxNt>), blocks, threads, 0, stream, d);
-  return hipGetLastError();
+  return wholeLines ? launch(helix_direct_exchange_kernel<kRanks, kWaves, kStatsPerThread, kAuxLoad, kAuxNtSc1>, blocks, threads, d, stream)
+                    : launch(helix_direct_exchange_kernel<kRanks, kWaves, kStatsPerThread, kAuxLoad, kAuxNt>, blocks, threads, d, stream);
 }
 
 template <int kRanks>
@@ -438,11 +440,9 @@ static hipError_t launch_combine_kernel(const KernelArgs& a, const uint64_t* bro
   d.groupedBlocks = blocks.x / (8 * d.xcdGroup) * (8 * d.xcdGroup);
   // a result that fits beside its inputs is written through (T = 256: 6.8 -> 6.5 us); one behind a stream of inputs is not
   // (T = 128, 16 heads of 512: 27.1, written through 27.6)
-  if (payload_bytes(a) > kStreamingBytes)
-    hipLaunchKernelGGL((helix_direct_combine_kernel<kDtype, kLanesPerSlot, kWords, kAuxNt, kAuxNt>), blocks, threads, 0, stream, d);
-  else
-    hipLaunchKernelGGL((helix_direct_combine_kernel<kDtype, kLanesPerSlot, kWords, kAuxNone, kAuxNtSc1>), blocks, threads, 0, stream, d);
-  return hipGetLastError();
+  return payload_bytes(a) > kStreamingBytes
+             ? launch(helix_direct_combine_kernel<kDtype, kLanesPerSlot, kWords, kAuxNt, kAuxNt>, blocks, threads, d, stream)
+             : launch(helix_direct_combine_kernel<kDtype, kLanesPerSlot, kWords, kAuxNone, kAuxNtSc1>, blocks, threads, d, stream);
 }
 
 template <int kLanesPerSlot>

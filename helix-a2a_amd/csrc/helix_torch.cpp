@@ -17,6 +17,7 @@
 #include <hip/hip_runtime_api.h>
 #include <torch/csrc/autograd/python_variable.h>
 
+#include <atomic>
 #include <chrono>
 #include <cstdlib>
 #include <mutex>
@@ -180,9 +181,16 @@ void fill_params(helix_a2a_params_t& p, int rank, int cp, int entries, const at:
   p.max_channel_count = maxChannels;
 }
 
-int device_max_channels(int cp) {
-  const int n = lib.maxChannelCount(cp, 0);
-  if (n < 0) raise_last("max_channel_count");
+// max_channel_count of the current device, asked once per (device, cp_size).
+int device_max_channels(const at::Device& device, int cp) {
+  static std::atomic<int> known[64][kMaxCp + 1];
+  std::atomic<int>& slot = known[device.index() & 63][cp];
+  int n = slot.load(std::memory_order_relaxed);
+  if (n == 0) {
+    n = lib.maxChannelCount(cp, 0);
+    if (n < 0) raise_last("max_channel_count");
+    slot.store(n, std::memory_order_relaxed);
+  }
   return n;
 }
 
@@ -298,7 +306,7 @@ PyObject* alltoall_loopback(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     try {
       require(!givenO || (PyList_GET_SIZE(givenO) == cp && PyList_GET_SIZE(givenS) == cp), "need one output pair per rank");
       helix_a2a_params_t params[kMaxCp];
-      const int maxChannels = device_max_channels(cp);
+      const int maxChannels = device_max_channels(device, cp);
       for (int r = 0; r < cp; ++r) {
         const at::Tensor &o = os.at(r), &s = ss.at(r);
         if (r > 0) {
@@ -374,7 +382,7 @@ PyObject* alltoall_combine_loopback(PyObject*, PyObject* const* args, Py_ssize_t
     if (returnLse) lse = Outputs(cp, {shape.entries, heads}, at::kFloat);
     helix_a2a_params_t params[kMaxCp];
     helix_a2a_combine_out_t out[kMaxCp];
-    const int maxChannels = device_max_channels(cp);
+    const int maxChannels = device_max_channels(device, cp);
     for (int r = 0; r < cp; ++r) {
       const at::Tensor &o = os.at(r), &s = ss.at(r);
       if (r > 0) {
@@ -427,7 +435,7 @@ PyObject* dcp_reduce(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     std::vector<at::Tensor> keep;  // contiguous copies, until the launch is enqueued
     helix_a2a_params_t params[kMaxCp];
     helix_a2a_combine_out_t out[kMaxCp];
-    const int maxChannels = device_max_channels(n);
+    const int maxChannels = device_max_channels(device, n);
     const int64_t lseSizes[2] = {b, h};
     for (int r = 0; r < n; ++r) {
       const at::Tensor *o = &os.at(r), *l = &ls.at(r);
@@ -694,7 +702,7 @@ PyObject* alltoall(PyObject*, PyObject* const* positional, Py_ssize_t nargs, PyO
       const OnDevice on(device);
       std::unique_ptr<Exchange> fresh(new Exchange);
       fresh->channels = env_channel_count();
-      fresh->maxChannels = device_max_channels(cp);
+      fresh->maxChannels = device_max_channels(device, cp);
       require(fresh->channels <= fresh->maxChannels, "alltoall: channel_count " + std::to_string(fresh->channels) +
                                                          " exceeds max_channel_count " + std::to_string(fresh->maxChannels));
       fresh->shape = shape;
