@@ -34,6 +34,8 @@ __device__ __forceinline__ void report_broken(const DirectCommon& a) {
   if (threadIdx.x % kWaveLanes == 0) atomicOr(a.status, kStatusBrokenWorkspace);
 }
 
+constexpr int kXcdRun = 64;  // consecutive workgroups' worth of payload one XCD takes, at most
+
 using GlobalPiece = __attribute__((address_space(1))) u32x2;
 
 // One workgroup moves kPerThread consecutive statistics pieces a thread in the order (entry, receiver, sender,
@@ -89,12 +91,23 @@ __device__ __forceinline__ void move_statistics(const DirectExchangeArgs<kRanks>
 // measured 0-4 % slower from 64 MB up and the same below). Groups of 2^groupShift consecutive wavefronts take
 // consecutive accesses of one pair, consecutive groups consecutive receivers, so that the launch sweeps all tensors in
 // order.
+//
+// Workgroups of four wavefronts run on the XCDs in runs of 64 consecutive ones. Neighbouring pairs read neighbouring rows
+// of a sender and write neighbouring rows of a receiver, and where a row is no whole number of lines they share the
+// lines between them: on XCDs of their own each of the two fetched the line and wrote its part of it. Three sets of
+// tensors in rotation: cp = 12, rows of 192 bytes, 73 MB 28.0 -> 24.8 us, of 480 bytes, 65 MB 23.3 -> 22.6; cp = 16, rows
+// of 160 bytes, 11 MB 6.8 -> 5.8; cp = 8, rows of 480 bytes, 32 MB 13.1 -> 12.6. Rows of whole lines only keep their
+// statistics' neighbours and their place in the sweep: 2 KiB, 34 MB 11.8 -> 11.5, cp = 16, 512 bytes, 134 MB 43.5 -> 43.3,
+// 640 bytes, 34 MB 11.7 -> 11.9. Runs of 8, 16 or 32 are within 2 % of that, but for the 160 bytes (6.5, 6.5, 5.5).
+// Workgroups of one wavefront stay as dispatched: rows of 16 KiB, 134 MB 42.6 us, in runs of 8 44.5, of 64 48.7.
 template <int kRanks, int kWaves, int kStatsPerThread, int kAuxLoad, int kAuxStore>
 __global__ __launch_bounds__(kWaves * kWaveLanes) void helix_direct_exchange_kernel(DirectExchangeArgs<kRanks> a) {
   __shared__ uint64_t from[kRanks], to[kRanks];
   if (blockIdx.x < a.statsBlocks) return move_statistics<kRanks, kWaves * kWaveLanes, kStatsPerThread>(a, from, to);
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWaveLanes);
-  const uint32_t w = (blockIdx.x - a.statsBlocks) * kWaves + wave;
+  uint32_t block = blockIdx.x - a.statsBlocks;
+  if (kWaves > 1 && block < a.groupedBlocks) block = static_cast<uint32_t>(xcd_grouped(static_cast<int>(block), a.xcdGroup));
+  const uint32_t w = block * kWaves + wave;
   if (w >= a.waves) return;
   const uint32_t pairs = w >> a.groupShift;
   const uint32_t t = fast_div_by(pairs, a.byCp);
@@ -122,7 +135,6 @@ __global__ __launch_bounds__(kWaves * kWaveLanes) void helix_direct_exchange_ker
 // 20.9 -> 5.5 us, T = 128, 16 heads of 512 71 -> 25.5 us (6.0 TB/s), cp = 16, T = 1024, 2 heads of 128 73 -> 25.7 us.
 
 constexpr int kCombineWaves = 4;  // wavefronts of a workgroup
-constexpr int kXcdRun = 64;       // consecutive workgroups' worth of pieces one XCD takes, at most
 
 // Pieces of kWords * 2 elements.
 template <int kDtype, int kWords>
@@ -354,6 +366,13 @@ static hipError_t launch(void (*kernel)(Args), dim3 blocks, dim3 threads, Args& 
   void* params[] = {&args};
   return hipLaunchKernel(reinterpret_cast<const void*>(kernel), blocks, threads, params, 0, stream);
 }
+// Whole tiles of eight runs; what is left of the launch stays as dispatched, and runs are shorter in launches of fewer
+// than eight.
+static void set_xcd_runs(DirectCommon& d, uint32_t blocks) {
+  d.xcdGroup = kXcdRun;
+  while (d.xcdGroup > 1 && 8u * d.xcdGroup > blocks) d.xcdGroup /= 2;
+  d.groupedBlocks = blocks / (8 * d.xcdGroup) * (8 * d.xcdGroup);
+}
 static uint64_t payload_bytes(const KernelArgs& a) { return static_cast<uint64_t>(a.cpSize) * a.sendBytes0; }
 
 template <int kRanks, int kWaves, int kStatsPerThread, int kAuxLoad>
@@ -362,7 +381,9 @@ static hipError_t launch_exchange_kernel(DirectExchangeArgs<kRanks>& d, uint32_t
   const uint32_t group = 1u << d.groupShift;
   d.statsBlocks = (d.pieces + kPiecesPerBlock - 1) / kPiecesPerBlock;
   d.waves = (chunks + group - 1) / group * group * d.cpSize * d.cpSize;
-  const dim3 blocks(d.statsBlocks + (d.waves + kWaves - 1) / kWaves), threads(kWaves * kWaveLanes);
+  const uint32_t payloadBlocks = (d.waves + kWaves - 1) / kWaves;
+  set_xcd_runs(d, payloadBlocks);
+  const dim3 blocks(d.statsBlocks + payloadBlocks), threads(kWaves * kWaveLanes);
   return wholeLines ? launch(helix_direct_exchange_kernel<kRanks, kWaves, kStatsPerThread, kAuxLoad, kAuxNtSc1>, blocks, threads, d, stream)
                     : launch(helix_direct_exchange_kernel<kRanks, kWaves, kStatsPerThread, kAuxLoad, kAuxNt>, blocks, threads, d, stream);
 }
@@ -435,9 +456,7 @@ static hipError_t launch_combine_kernel(const KernelArgs& a, const uint64_t* bro
   d.lseBase2 = a.lseBase2;
   d.waves = (d.outPieces + kWaveLanes - 1) / kWaveLanes * d.cpSize;  // at most 2^22: a rank's output is < 2 GiB / cp
   const dim3 blocks((d.waves + kCombineWaves - 1) / kCombineWaves), threads(kCombineWaves * kWaveLanes);
-  d.xcdGroup = kXcdRun;
-  while (d.xcdGroup > 1 && 8u * d.xcdGroup > blocks.x) d.xcdGroup /= 2;
-  d.groupedBlocks = blocks.x / (8 * d.xcdGroup) * (8 * d.xcdGroup);
+  set_xcd_runs(d, blocks.x);
   // a result that fits beside its inputs is written through (T = 256: 6.8 -> 6.5 us); one behind a stream of inputs is not
   // (T = 128, 16 heads of 512: 27.1, written through 27.6)
   return payload_bytes(a) > kStreamingBytes

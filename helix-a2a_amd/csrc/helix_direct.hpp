@@ -28,6 +28,8 @@ struct DirectCommon {
   uint32_t sendBytes0, recvBytes0;    // extent of each partial_o and result tensor (< 2 GiB), the range of its buffer descriptor
   uint32_t waves;                     // wavefronts of the launch that move partial_o
   FastDiv byCp;
+  int xcdGroup;            // consecutive workgroups' worth of partial_o that one XCD takes (xcd_grouped) ...
+  uint32_t groupedBlocks;  // ... in the first so many workgroups that move partial_o, whole tiles of it
 };
 
 template <int kRanks>
@@ -55,8 +57,6 @@ struct DirectCombine {
   uint32_t headPieces;  // of a head
   uint32_t heads;       // heads of a row
   FastDiv byHeadPieces, byHeads;
-  int xcdGroup;            // consecutive workgroups' worth of pieces that one XCD takes (xcd_grouped) ...
-  uint32_t groupedBlocks;  // ... in the first so many workgroups, whole tiles of it
   int statsMode, lseBase2;
 };
 

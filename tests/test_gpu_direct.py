@@ -59,6 +59,10 @@ CASES = [
     (8, 64, 1024, 16, 64),      # whole lines
     (8, 64, 1024, 16, 4),       # ... but outputs that start inside a line
     (32, 9, 128, 8, 0),
+    (2, 7, 512, 2, 0),          # seven workgroups: none to a run
+    (2, 9, 512, 2, 0),          # nine: runs of one, and a rest as dispatched
+    (2, 512, 512, 2, 0),        # runs of sixty-four to an XCD
+    (2, 519, 512, 2, 0),        # ... and a rest
     (8, 385, 1024, 16, 0),      # 50 MB: workgroups of one wavefront
     (9, 311, 1032, 2, 0),       # ... ragged, rows that are no whole lines
     (8, 3100, 128, 2, 0),       # ... but not for rows shorter than an access
