@@ -15,6 +15,7 @@
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <atomic>
@@ -62,6 +63,8 @@ PyObject* guarded(F&& body) {
   try {
     return body();
   } catch (const PythonError&) {
+  } catch (const c10::OutOfMemoryError& e) {  // torch.cuda.OutOfMemoryError, as from torch.empty
+    PyErr_SetString(THPException_OutOfMemoryError, e.what_without_backtrace());
   } catch (const c10::Error& e) {
     PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
   } catch (const std::exception& e) {

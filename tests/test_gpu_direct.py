@@ -175,3 +175,22 @@ def test_direct_combine(hx, ops, cp, entries, heads, d, dtype, mode, base2):
         finite = np.isfinite(want_lse)
         worst = float(np.max(np.abs(got_lse[finite] - want_lse[finite]) / np.maximum(np.abs(want_lse[finite]), 4.0), initial=0.0))
         assert worst <= 2.0 ** -17, f"log-sum-exp of rank {r}: {worst}"
+
+
+def test_out_of_memory_is_reported_as_torch_reports_it(hx):
+    ws = workspace(hx, 2)
+    ins_o = [torch.zeros(4096, 2, 8192, device="cuda", dtype=torch.bfloat16) for _ in range(2)]
+    ins_s = [torch.zeros(4096, 2, 2, device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    free, total = torch.cuda.mem_get_info()
+    torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)  # the outputs take 256 MiB
+    try:
+        for call in (lambda: hx.alltoall_loopback(ins_o, ins_s, ws), lambda: hx.alltoall(ins_o[0], ins_s[0], ws, 0, 2)):
+            with pytest.raises(torch.cuda.OutOfMemoryError):
+                call()
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    outs_o, _ = hx.alltoall_loopback(ins_o, ins_s, ws)  # nothing is left behind
+    torch.cuda.synchronize()
+    assert all(not t.any() for t in outs_o)
