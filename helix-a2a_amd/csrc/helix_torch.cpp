@@ -21,6 +21,7 @@
 #include <atomic>
 #include <chrono>
 #include <cstdlib>
+#include <exception>
 #include <mutex>
 #include <stdexcept>
 #include <string>
@@ -63,8 +64,8 @@ PyObject* guarded(F&& body) {
   try {
     return body();
   } catch (const PythonError&) {
-  } catch (const c10::OutOfMemoryError& e) {  // torch.cuda.OutOfMemoryError, as from torch.empty
-    PyErr_SetString(THPException_OutOfMemoryError, e.what_without_backtrace());
+  } catch (const c10::OutOfMemoryError&) {  // torch.cuda.OutOfMemoryError, as from torch.empty
+    torch::translate_exception_to_python(std::current_exception());
   } catch (const c10::Error& e) {
     PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
   } catch (const std::exception& e) {

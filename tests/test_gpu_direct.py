@@ -1,5 +1,7 @@
 """GPU tests of the loopback calls that copy between the ranks' tensors directly (no channel count given), at the sizes
 where their kernels change course, bit for bit against the oracle's single strided copy."""
+import gc
+
 import pytest
 import torch
 
@@ -178,12 +180,15 @@ def test_direct_combine(hx, ops, cp, entries, heads, d, dtype, mode, base2):
 
 
 def test_out_of_memory_is_reported_as_torch_reports_it(hx):
+    _WS.clear()
+    gc.collect()
+    torch.cuda.empty_cache()  # no large block of an earlier test to carve the tensors out of
     ws = workspace(hx, 2)
     ins_o = [torch.zeros(4096, 2, 8192, device="cuda", dtype=torch.bfloat16) for _ in range(2)]
     ins_s = [torch.zeros(4096, 2, 2, device="cuda") for _ in range(2)]
     torch.cuda.synchronize()
     torch.cuda.empty_cache()
-    free, total = torch.cuda.mem_get_info()
+    _, total = torch.cuda.mem_get_info()
     torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)  # the outputs take 256 MiB
     try:
         for call in (lambda: hx.alltoall_loopback(ins_o, ins_s, ws), lambda: hx.alltoall(ins_o[0], ins_s[0], ws, 0, 2)):
