@@ -211,20 +211,22 @@ struct Outputs {
     storage = c10::Storage(c10::make_intrusive<c10::StorageImpl>(c10::StorageImpl::use_byte_size_t(), static_cast<size_t>(cp * numel) * dtype.itemsize(),
                                                                  c10::hip::HIPCachingAllocatorMasqueradingAsCUDA::get(), /*resizable=*/true));
   }
-  at::Tensor slice(int r) const {
+  at::Tensor slice(int r) const { return slice(r, sizes); }
+  at::Tensor slice(int r, at::IntArrayRef shape) const {
     at::Tensor t = at::detail::make_tensor<c10::TensorImpl>(c10::Storage(storage), c10::DispatchKeySet(c10::DispatchKey::CUDA), dtype);
     t.unsafeGetTensorImpl()->set_storage_offset(r * numel);
-    t.unsafeGetTensorImpl()->set_sizes_contiguous(sizes);
+    t.unsafeGetTensorImpl()->set_sizes_contiguous(shape);
     return t;
   }
   void* data(int r) const { return static_cast<char*>(storage.mutable_data()) + r * numel * static_cast<int64_t>(dtype.itemsize()); }
 };
 
-PyObject* wrap_slices(const Outputs& out, int cp) {
+// The slices as a list; those of the ranks in `otherRanks` have the sizes `other`.
+PyObject* wrap_slices(const Outputs& out, int cp, uint32_t otherRanks = 0, at::IntArrayRef other = {}) {
   PyObject* list = PyList_New(cp);
   if (!list) throw PythonError{};
   for (int r = 0; r < cp; ++r) {
-    PyObject* t = THPVariable_Wrap(out.slice(r));
+    PyObject* t = THPVariable_Wrap((otherRanks >> r) & 1u ? out.slice(r, other) : out.slice(r));
     if (!t) {
       Py_DECREF(list);
       throw PythonError{};
@@ -349,8 +351,9 @@ PyObject* alltoall_loopback(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
 }
 
 // The combined outputs of all ranks (and their log-sum-exps) as Python lists.
-PyObject* combine_result(const Outputs& combined, const Outputs& lse, int cp, bool returnLse) {
-  PyObject* first = wrap_slices(combined, cp);
+PyObject* combine_result(const Outputs& combined, const Outputs& lse, int cp, bool returnLse, uint32_t otherRanks = 0,
+                         at::IntArrayRef other = {}) {
+  PyObject* first = wrap_slices(combined, cp, otherRanks, other);
   return returnLse ? pair(first, wrap_slices(lse, cp)) : first;
 }
 
@@ -378,11 +381,9 @@ PyObject* alltoall_combine_loopback(PyObject*, PyObject* const* args, Py_ssize_t
     const at::Device device = ws.device();
     const OnDevice on(device);
 
-    Outputs combined, lse;
-    if (o0.dim() == 4 && o0.size(1) == cp && o0.size(2) == heads)
-      combined = Outputs(cp, {shape.entries, heads, shape.row0 / heads}, o0.scalar_type());
-    else
-      combined = Outputs(cp, {shape.entries, shape.row0}, o0.scalar_type());
+    Outputs combined(cp, {shape.entries, shape.row0}, o0.scalar_type()), lse;
+    const int64_t perHead[3] = {shape.entries, heads, shape.row0 / heads};  // what a rank that passes [T, cp, H/cp, D] gets
+    uint32_t perHeadRanks = 0;
     if (returnLse) lse = Outputs(cp, {shape.entries, heads}, at::kFloat);
     helix_a2a_params_t params[kMaxCp];
     helix_a2a_combine_out_t out[kMaxCp];
@@ -392,10 +393,15 @@ PyObject* alltoall_combine_loopback(PyObject*, PyObject* const* args, Py_ssize_t
       if (r > 0) {
         require(o.is_cuda(), "partial_o must be on the GPU");
         require(s.is_cuda(), "softmax_stats must be on the GPU");
-        require(same_pair(o, s, o0, s0), "all ranks must exchange tensors of one shape and dtype");
+        if (!same_pair(o, s, o0, s0)) {  // other dimensions of the same rows will do
+          const Shape other = check_pair(o, s, cp);
+          require(other.entries == shape.entries && other.row0 == shape.row0 && other.row1 == shape.row1 && o.scalar_type() == o0.scalar_type(),
+                  "all ranks must exchange tensors of one shape and dtype");
+        }
         require(o.is_contiguous(), "partial_o must be contiguous");
         require(s.is_contiguous(), "softmax_stats must be contiguous");
       }
+      if (o.dim() == 4 && o.size(1) == cp && o.size(2) == heads) perHeadRanks |= 1u << r;
       require(o.device() == device && s.device() == device, "all tensors must live on one device");
       fill_params(params[r], r, cp, shape.entries, o, s, nullptr, nullptr, shape.row0, shape.row1, ws, channels, maxChannels);
       out[r].combined = combined.data(r);
@@ -404,7 +410,7 @@ PyObject* alltoall_combine_loopback(PyObject*, PyObject* const* args, Py_ssize_t
     const hipStream_t stream = current_stream(device);
     const int dtype = o0.scalar_type() == at::kBFloat16 ? HELIX_A2A_DTYPE_BF16 : HELIX_A2A_DTYPE_FP16;
     launch("alltoall_combine_loopback", [&] { return lib.combine(params, out, cp, mode, dtype, stream); });
-    return combine_result(combined, lse, cp, returnLse != 0);
+    return combine_result(combined, lse, cp, returnLse != 0, perHeadRanks, perHead);
   });
 }
 

@@ -199,3 +199,21 @@ def test_out_of_memory_is_reported_as_torch_reports_it(hx):
     outs_o, _ = hx.alltoall_loopback(ins_o, ins_s, ws)  # nothing is left behind
     torch.cuda.synchronize()
     assert all(not t.any() for t in outs_o)
+
+
+def test_combine_takes_ranks_whose_tensors_have_other_dimensions(hx, ops):
+    """[E, cp, heads * D] of one rank and [E, cp, heads, D] of another hold the same rows; each gets its own form back."""
+    cp, entries, heads, d = 2, 5, 3, 64
+    ws = workspace(hx, cp)
+    flat_o = [torch.randn(entries, cp, heads * d, device="cuda").to(torch.bfloat16) for _ in range(cp)]
+    flat_s = [torch.rand(entries, cp, heads * 2, device="cuda") + 1 for _ in range(cp)]
+    want, want_lse = hx.alltoall_combine_loopback(flat_o, flat_s, ws, ops.STATS_MAX_SUM, True)
+    for four_d in ((True, False), (False, True), (True, True)):
+        o = [t.view(entries, cp, heads, d) if f else t for t, f in zip(flat_o, four_d)]
+        s = [t.view(entries, cp, heads, 2) if f else t for t, f in zip(flat_s, four_d)]
+        got, got_lse = hx.alltoall_combine_loopback(o, s, ws, ops.STATS_MAX_SUM, True)
+        for r, f in enumerate(four_d):
+            assert got[r].shape == ((entries, heads, d) if f else (entries, heads * d)) and got[r].is_contiguous()
+            assert torch.equal(got[r].view(want[r].shape), want[r]) and torch.equal(got_lse[r], want_lse[r])
+    with pytest.raises(RuntimeError, match="one shape and dtype"):
+        hx.alltoall_combine_loopback([flat_o[0], flat_o[1][:4].contiguous()], [flat_s[0], flat_s[1][:4].contiguous()], ws)
