@@ -81,6 +81,18 @@ int as_int(PyObject* o) {
   return static_cast<int>(v);
 }
 
+// channel_count: whatever int() takes.
+int as_channels(PyObject* o) {
+  if (PyLong_Check(o)) return as_int(o);
+  PyObject* v = PyNumber_Long(o);
+  if (!v) throw PythonError{};
+  const long n = PyLong_AsLong(v);
+  Py_DECREF(v);
+  if (n == -1 && PyErr_Occurred()) throw PythonError{};
+  require(n >= INT32_MIN && n <= INT32_MAX, "integer argument out of range");
+  return static_cast<int>(n);
+}
+
 const at::Tensor& as_tensor(PyObject* o, const char* message) {
   require(THPVariable_Check(o), message);
   return THPVariable_Unpack(o);
@@ -285,7 +297,7 @@ PyObject* alltoall_loopback(PyObject*, PyObject* const* args, Py_ssize_t nargs) 
     require(cp >= 1 && cp <= kMaxCp && ss.size() == cp, "need one partial_o and one softmax_stats tensor per rank");
     const at::Tensor& ws = as_tensor(args[2], "workspace must be on the GPU");
     check_workspace(ws, cp);
-    const int channels = as_int(args[3]);
+    const int channels = as_channels(args[3]);
     const at::Tensor &o0 = os.at(0), &s0 = ss.at(0);
     const Shape shape = check_pair(o0, s0, cp);
     const at::Device device = ws.device();
@@ -372,7 +384,7 @@ PyObject* alltoall_combine_loopback(PyObject*, PyObject* const* args, Py_ssize_t
     if (returnLse < 0) throw PythonError{};
     const at::Tensor& ws = as_tensor(args[2], "workspace must be on the GPU");
     check_workspace(ws, cp);
-    const int channels = as_int(args[5]);
+    const int channels = as_channels(args[5]);
     const at::Tensor &o0 = os.at(0), &s0 = ss.at(0);
     const Shape shape = check_pair(o0, s0, cp);
     const int heads = mode == HELIX_A2A_STATS_LSE_PACKED ? shape.row1 : shape.row1 / 2;
@@ -437,7 +449,7 @@ PyObject* dcp_reduce(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     require(b <= INT32_MAX && hp * d <= INT32_MAX / 2, "cp_attn_out is too large");
     const int returnLse = PyObject_IsTrue(args[3]), base2 = PyObject_IsTrue(args[5]);
     if (returnLse < 0 || base2 < 0) throw PythonError{};
-    const int channels = as_int(args[4]);
+    const int channels = as_channels(args[4]);
     const OnDevice on(device);
 
     Outputs combined(n, {b, hp, d}, o0.scalar_type()), lse;

@@ -217,3 +217,42 @@ def test_combine_takes_ranks_whose_tensors_have_other_dimensions(hx, ops):
             assert torch.equal(got[r].view(want[r].shape), want[r]) and torch.equal(got_lse[r], want_lse[r])
     with pytest.raises(RuntimeError, match="one shape and dtype"):
         hx.alltoall_combine_loopback([flat_o[0], flat_o[1][:4].contiguous()], [flat_s[0], flat_s[1][:4].contiguous()], ws)
+
+
+@pytest.mark.parametrize("channels", [3.0, "3", 0.0])
+def test_channel_count_takes_what_int_takes(hx, channels):
+    cp = 2
+    ws = workspace(hx, cp)
+    ins_o = [torch.randn(5, cp, 2 * 32, device="cuda").to(torch.bfloat16) for _ in range(cp)]
+    ins_s = [torch.rand(5, cp, 2 * 2, device="cuda") + 1 for _ in range(cp)]
+    outs_o, _ = hx.alltoall_loopback(ins_o, ins_s, ws, channel_count=channels)
+    combined = hx.alltoall_combine_loopback(ins_o, ins_s, ws, channel_count=channels)
+    reduced = hx.dcp_a2a_lse_reduce([t.view(5, 2 * cp, 32) for t in ins_o], [t[:, :, :2].reshape(5, 2 * cp) for t in ins_s], ws,
+                                    channel_count=channels)
+    for r in range(cp):
+        assert torch.equal(outs_o[r], torch.stack([ins_o[s][:, r] for s in range(cp)], 1))
+        assert combined[r].shape == (5, 64) and reduced[r].shape == (5, 2, 32)
+    with pytest.raises(RuntimeError, match="exceeds max_channel_count"):
+        hx.alltoall_loopback(ins_o, ins_s, ws, channel_count=1e9)
+    with pytest.raises(TypeError):
+        hx.alltoall_loopback(ins_o, ins_s, ws, channel_count=None)
+
+
+@pytest.mark.parametrize("shift", [4, 60])
+@pytest.mark.parametrize("d", [40, 36])
+def test_inputs_that_start_inside_a_line(hx, ops, shift, d):
+    """Tensors are asked to start on 8 bytes; 16-byte accesses from such a start give what they give from a line's."""
+    cp, entries, heads = 5, 33, 4
+    ws = workspace(hx, cp)
+    ins_o = [torch.randn(entries, cp, heads * d, device="cuda").to(torch.bfloat16) for _ in range(cp)]
+    ins_s = [torch.rand(entries, cp, heads * 2, device="cuda") + 1 for _ in range(cp)]
+
+    def shifted(t):
+        raw = torch.empty(t.numel() + shift, dtype=t.dtype, device="cuda")
+        raw[shift:] = t.flatten()
+        return raw[shift:].view(t.shape)
+
+    for call in (lambda o, s: sum(hx.alltoall_loopback(o, s, ws), []),
+                 lambda o, s: sum(hx.alltoall_combine_loopback(o, s, ws, ops.STATS_MAX_SUM, True), [])):
+        for got, want in zip(call([shifted(t) for t in ins_o], [shifted(t) for t in ins_s]), call(ins_o, ins_s)):
+            assert torch.equal(got, want)
