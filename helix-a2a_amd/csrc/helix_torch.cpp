@@ -739,8 +739,9 @@ PyObject* alltoall(PyObject*, PyObject* const* positional, Py_ssize_t nargs, PyO
     struct Owner {
       Group* group;
       Exchange* ex;
+      bool handedOn = false;
       ~Owner() {
-        if (group->ex != ex) delete ex;
+        if (!handedOn && group->ex != ex) delete ex;
         Py_DECREF(group);
       }
     } owner{group, ex};
@@ -766,27 +767,24 @@ PyObject* alltoall(PyObject*, PyObject* const* positional, Py_ssize_t nargs, PyO
     ex->stream[rank] = stream;
     ex->called |= 1u << rank;
     ex->calls += 1;
-    PyObject* outO = THPVariable_Wrap(ex->outO.slice(rank));
+    const at::Tensor sliceO = ex->outO.slice(rank), sliceS = ex->outS.slice(rank);
+    // The group is up to date before the next Python object is made: making one can collect garbage, and other threads
+    // may run meanwhile and call for their ranks. From here on `ex` is theirs too unless this was the last rank.
+    const bool last = ex->calls == cp;
+    owner.handedOn = !last;
+    group->ex = last ? nullptr : ex;  // (the next exchange may start while this one is being enqueued)
+    if (last) {
+      const OnDevice on(device);
+      flush(*ex, cp, stream);
+    }
+    PyObject* outO = THPVariable_Wrap(sliceO);
     if (!outO) throw PythonError{};
-    PyObject* outS = THPVariable_Wrap(ex->outS.slice(rank));
+    PyObject* outS = THPVariable_Wrap(sliceS);
     if (!outS) {
       Py_DECREF(outO);
       throw PythonError{};
     }
-    PyObject* result = pair(outO, outS);
-    if (ex->calls < cp) {
-      group->ex = ex;
-      return result;
-    }
-    group->ex = nullptr;  // the next exchange may start while this one is being enqueued
-    try {
-      const OnDevice on(device);
-      flush(*ex, cp, stream);
-    } catch (...) {
-      Py_DECREF(result);
-      throw;
-    }
-    return result;
+    return pair(outO, outS);
   });
 }
 

@@ -256,3 +256,48 @@ def test_inputs_that_start_inside_a_line(hx, ops, shift, d):
                  lambda o, s: sum(hx.alltoall_combine_loopback(o, s, ws, ops.STATS_MAX_SUM, True), [])):
         for got, want in zip(call([shifted(t) for t in ins_o], [shifted(t) for t in ins_s]), call(ins_o, ins_s)):
             assert torch.equal(got, want)
+
+
+def test_ranks_of_several_threads_with_collections_in_between(hx):
+    """A collection may start wherever a call makes a Python object, and whatever it runs may let the other threads in."""
+    import threading
+    import time
+
+    cp, steps = 4, 12
+    ws = workspace(hx, cp)
+    ins_o = [[torch.randn(5, cp, 64, device="cuda").to(torch.bfloat16) for _ in range(cp)] for _ in range(steps)]
+    ins_s = [[torch.rand(5, cp, 2, device="cuda") for _ in range(cp)] for _ in range(steps)]
+    got = [[None] * cp for _ in range(steps)]
+    turn, failures = threading.Barrier(cp), []
+    torch.cuda.synchronize()
+
+    def rank(r):
+        try:
+            for i in range(steps):
+                turn.wait(60)
+                got[i][r] = hx.alltoall(ins_o[i][r], ins_s[i][r], ws, r, cp)
+        except Exception as e:  # noqa: BLE001
+            failures.append(e)
+            turn.abort()
+
+    def yielding(phase, info):
+        time.sleep(1e-3)
+
+    threshold = gc.get_threshold()
+    gc.callbacks.append(yielding)
+    gc.set_threshold(1)
+    try:
+        threads = [threading.Thread(target=rank, args=(r,)) for r in range(cp)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        gc.set_threshold(*threshold)
+        gc.callbacks.remove(yielding)
+    assert not failures, failures
+    torch.cuda.synchronize()
+    for i in range(steps):
+        for r in range(cp):
+            assert torch.equal(got[i][r][0], torch.stack([ins_o[i][s][:, r] for s in range(cp)], 1)), (i, r)
+            assert torch.equal(got[i][r][1], torch.stack([ins_s[i][s][:, r] for s in range(cp)], 1)), (i, r)
