@@ -4,8 +4,8 @@
 // exchange is a copy in rows: what bounds it is the memory system, and from
 // where the ranks' memory is in reach the only work is to read every byte once
 // and write it once. Against the same exchange through FIFO lines (write, read
-// back): cp = 8, T = 256, rows of 2 KiB 24 -> 10 us, rows of 16 KiB at T = 128
-// 83 -> 46 us (5.9 TB/s, a plain copy of 1 GiB reaches 6.2), cp = 16, T = 1024,
+// back): cp = 8, T = 256, rows of 2 KiB 24 -> 11 us, rows of 16 KiB at T = 128
+// 83 -> 43 us (6.3 TB/s, a plain copy of 1 GiB reaches 6.2), cp = 16, T = 1024,
 // rows of 512 bytes 93 -> 43 us.
 #include "helix_direct.hpp"
 #include "helix_element.hpp"
